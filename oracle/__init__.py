@@ -38,7 +38,7 @@ def build(ref: bool | None = None, fast: bool = True) -> None:
     """Compile liboracle.so (and the reference pieces when the reference is mounted)."""
     targets = ["liboracle.so"] + (["liboracle_fast.so"] if fast else [])
     if ref is None:
-        ref = os.path.isdir(REF_ROOT)
+        ref = os.path.isfile(os.path.join(REF_ROOT, "eig3", "eig3.cpp"))  # mounted, and not an empty folder
     if ref:
         targets.append("ref")
     subprocess.run(["make", "-s", "-C", HERE] + targets, check=True)
