@@ -7,7 +7,8 @@
 // Level-synchronous: the nodes of one depth, across every mesh of the
 // batch, are one launch, one 64-lane workgroup per node at a time (levels
 // are launched in batches; each launch reads its node range from the
-// previous one).  Within a node:
+// previous one); nodes of more than BIG_TRIS triangles are spread over the
+// chip tile by tile instead (bigbuild.hpp).  Within a node:
 //   * the distinct-point check is a wave ballot;
 //   * the mean and the six covariance sums are SEQUENTIAL double chains in
 //     point order (the reference's std::accumulate / std::inner_product),
@@ -48,7 +49,10 @@ struct LevelArgs {
     float* pos_fin;
     uint32_t* id_fin;
     unsigned int* mesh_depth;
+    unsigned int* slack_bits;   // SLACK_REPS copies per mesh
+    unsigned int* radius_bits;  // one per mesh
     uint32_t leaf_max;
+    uint32_t big_min;           // nodes of more triangles than this take the tiled passes
 };
 
 constexpr int CHUNK = 256;                 // points per step of the sequential chains
@@ -214,6 +218,137 @@ __device__ __forceinline__ void load_tris(const float* __restrict__ P, uint32_t 
     }
 }
 
+// The box of a node from its axes and the extents along them
+// (OBB::CreateAABBfromPoints' tail and OBB.cpp:74-89).
+__device__ inline void box_of_extents(const double* ax, const double* lo, const double* hi, float* box12) {
+    double cx = 0.0, cy = 0.0, cz = 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        double delta = (hi[q] - lo[q]) + 2.0 * double(FLT_EPSILON);
+        double mid = (hi[q] + lo[q]) / 2.0;
+        cx = cx + mid * ax[3 * q];
+        cy = cy + mid * ax[3 * q + 1];
+        cz = cz + mid * ax[3 * q + 2];
+        double half = delta / 2.0;
+        box12[3 + 3 * q] = float(half * ax[3 * q]);
+        box12[4 + 3 * q] = float(half * ax[3 * q + 1]);
+        box12[5 + 3 * q] = float(half * ax[3 * q + 2]);
+    }
+    box12[0] = float(cx);
+    box12[1] = float(cy);
+    box12[2] = float(cz);
+}
+
+// OBB::EmptyOBB (OBB.cpp:168-178) at a point.
+__device__ inline Box empty_box(f3 c) {
+    const float e = FLT_EPSILON;
+    Box b;
+    b.c = c;
+    b.u = mk(e, 0.f, 0.f);
+    b.v = mk(0.f, e, 0.f);
+    b.w = mk(0.f, 0.f, e);
+    return b;
+}
+
+// How far a point lies outside a box meant to hold it: its coordinates in the
+// side vectors are its offset dotted with the dual basis (v x w, w x u,
+// u x v) / det(u, v, w).  A mesh's slack is the largest excess of any point
+// over any box above it; it is taken where the node's triangles are read for
+// its split anyway, as a pass of its own read every level's triangles again
+// (one wavefront per node: 1.8 ms for a level load with a 198,450-triangle
+// terrain).
+struct Excess {
+    double c[3], du[3], dv[3], dw[3], lu, lv, lw;
+    bool flat;
+    __device__ explicit Excess(const Box& b) {
+        const double u[3] = {b.u.x, b.u.y, b.u.z}, v[3] = {b.v.x, b.v.y, b.v.z}, w[3] = {b.w.x, b.w.y, b.w.z};
+        auto cross = [](const double* a, const double* q, double* o) {
+            o[0] = a[1] * q[2] - a[2] * q[1];
+            o[1] = a[2] * q[0] - a[0] * q[2];
+            o[2] = a[0] * q[1] - a[1] * q[0];
+        };
+        c[0] = b.c.x;
+        c[1] = b.c.y;
+        c[2] = b.c.z;
+        cross(v, w, du);
+        cross(w, u, dv);
+        cross(u, v, dw);
+        const double D = u[0] * du[0] + u[1] * du[1] + u[2] * du[2];
+        for (int k = 0; k < 3; ++k) {
+            du[k] = du[k] / D;
+            dv[k] = dv[k] / D;
+            dw[k] = dw[k] / D;
+        }
+        flat = !(fabs(D) > 0.0);
+        lu = sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+        lv = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+        lw = sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
+    }
+    __device__ __forceinline__ double of(const float* p) const {
+        if (flat) return INFINITY;
+        const double r[3] = {double(p[0]) - c[0], double(p[1]) - c[1], double(p[2]) - c[2]};
+        const double al = r[0] * du[0] + r[1] * du[1] + r[2] * du[2];
+        const double be = r[0] * dv[0] + r[1] * dv[1] + r[2] * dv[2];
+        const double ga = r[0] * dw[0] + r[1] * dw[1] + r[2] * dw[2];
+        return fmax(0.0, fabs(al) - 1.0) * lu + fmax(0.0, fabs(be) - 1.0) * lv + fmax(0.0, fabs(ga) - 1.0) * lw;
+    }
+    // the largest excess and squared norm over a triangle's corners
+    __device__ __forceinline__ void take(const float* t9, double& worst, double& rad2) const {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const float* p = t9 + 3 * k;
+            worst = fmax(worst, of(p));
+            rad2 = fmax(rad2, double(p[0]) * double(p[0]) + double(p[1]) * double(p[1]) + double(p[2]) * double(p[2]));
+        }
+    }
+};
+__device__ inline float round_up(double x) {  // to float, so that the bound stays an upper bound
+    float f = float(x);
+    if (double(f) < x) f = nextafterf(f, INFINITY);
+    return f;
+}
+// One of SLACK_REPS copies per mesh, so that a mesh's many nodes do not queue
+// on one address; the radius is the root's (sqrt is monotone: the root of
+// the largest square is the largest root).
+__device__ inline void post_excess(const LevelArgs& a, const BNode& nd, uint32_t rep, double worst, double rad2) {
+    atomicMax(&a.slack_bits[size_t(nd.mesh) * SLACK_REPS + (rep % SLACK_REPS)], __float_as_uint(round_up(worst)));
+    if (nd.level == 0) atomicMax(&a.radius_bits[nd.mesh], __float_as_uint(round_up(sqrt(rad2))));
+}
+
+// The children of a split node, appended to the next level.
+__device__ inline uint32_t append_kids(const LevelArgs& a, BNode* nd, uint32_t nl, uint32_t next_first,
+                                       unsigned int* next_count) {
+    const uint32_t beg = nd->beg, end = nd->end;
+    const uint32_t slot = next_first + atomicAdd(next_count, 2u);
+    BNode* k0 = &a.nodes[slot];
+    BNode* k1 = &a.nodes[slot + 1];
+    k0->mesh = nd->mesh; k0->beg = beg;      k0->end = beg + nl; k0->level = nd->level + 1; k0->flags = 0;
+    k1->mesh = nd->mesh; k1->beg = beg + nl; k1->end = end;      k1->level = nd->level + 1; k1->flags = 0;
+    nd->kid[0] = slot;
+    nd->kid[1] = slot + 1;
+    nd->flags = 0;
+    atomicMax(&a.mesh_depth[nd->mesh], nd->level + 1);
+    return slot;
+}
+
+// The split's three candidates, longest first (OBBtree.cpp:45-51), and their centre projections.
+__device__ inline void split_candidates(const Box& box, AxisCand (&cand)[3], float (&cp)[3]) {
+    cand[0] = {vlength(box.u), normalize(box.u)};
+    cand[1] = {vlength(box.v), normalize(box.v)};
+    cand[2] = {vlength(box.w), normalize(box.w)};
+    sort3_desc(cand);
+#pragma unroll
+    for (int ch = 0; ch < 3; ++ch) cp[ch] = dot(box.c, cand[ch].dir);
+}
+// The first candidate that leaves both sides non-empty, else -1: index halves (OBBtree.cpp:81-93).
+__device__ inline int split_pick(const uint32_t (&cnt)[3], uint32_t n) {
+    int pick = -1;
+#pragma unroll
+    for (int ch = 2; ch >= 0; --ch)
+        if (cnt[ch] != 0 && cnt[ch] != n) pick = ch;
+    return pick;
+}
+
 struct LevelShared {
     float raw[CHUNK * 3];
     double val[CHUNK * 6];
@@ -247,11 +382,7 @@ __device__ __forceinline__ void level_node(const LevelArgs& a, uint32_t ni, uint
     }
     Box box;
     if (npts == 0 || !multi) {
-        const float e = FLT_EPSILON;  // OBB::EmptyOBB (OBB.cpp:168-178)
-        box.c = npts ? mk(P[0], P[1], P[2]) : mk(0.f, 0.f, 0.f);
-        box.u = mk(e, 0.f, 0.f);
-        box.v = mk(0.f, e, 0.f);
-        box.w = mk(0.f, 0.f, e);
+        box = empty_box(npts ? mk(P[0], P[1], P[2]) : mk(0.f, 0.f, 0.f));
     } else {
         const double N = double(npts);
         double acc = stream_chain<3>(
@@ -332,26 +463,7 @@ __device__ __forceinline__ void level_node(const LevelArgs& a, uint32_t ni, uint
             wave_min_last(lo[q], loi[q]);
             wave_max_first(hi[q], hii[q]);
         }
-        if (lane == 0) {
-            double cx = 0.0, cy = 0.0, cz = 0.0;
-            float side[3][3];
-            for (int q = 0; q < 3; ++q) {
-                double delta = (hi[q] - lo[q]) + 2.0 * double(FLT_EPSILON);
-                double mid = (hi[q] + lo[q]) / 2.0;
-                cx = cx + mid * ax[3 * q];
-                cy = cy + mid * ax[3 * q + 1];
-                cz = cz + mid * ax[3 * q + 2];
-                double half = delta / 2.0;
-                side[q][0] = float(half * ax[3 * q]);
-                side[q][1] = float(half * ax[3 * q + 1]);
-                side[q][2] = float(half * ax[3 * q + 2]);
-            }
-            S.box[0] = float(cx);
-            S.box[1] = float(cy);
-            S.box[2] = float(cz);
-            for (int q = 0; q < 3; ++q)
-                for (int c = 0; c < 3; ++c) S.box[3 + 3 * q + c] = side[q][c];
-        }
+        if (lane == 0) box_of_extents(ax, lo, hi, S.box);
         wave_sync();
         box = box_from12(S.box);
     }
@@ -360,10 +472,29 @@ __device__ __forceinline__ void level_node(const LevelArgs& a, uint32_t ni, uint
         nd->surf = surface(box);
     }
 
+    const Excess ex(box);
+    double worst = 0.0, rad2 = 0.0;
+    auto post = [&]() {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            worst = fmax(worst, __shfl_xor(worst, off, 64));
+            rad2 = fmax(rad2, __shfl_xor(rad2, off, 64));
+        }
+        if (lane == 0) post_excess(a, *nd, ni, worst, rad2);
+    };
+
     // ---- leaf: park the triangles in their final slots ----
     if (n <= a.leaf_max) {
-        for (uint32_t t = lane; t < 9 * n; t += 64) a.pos_fin[size_t(beg) * 9 + t] = P[t];
-        for (uint32_t t = lane; t < n; t += 64) a.id_fin[beg + t] = a.id_in[beg + t];
+        for (uint32_t t = lane; t < n; t += 64) {
+            float T[9];
+#pragma unroll
+            for (int q = 0; q < 9; ++q) T[q] = P[size_t(t) * 9 + q];
+#pragma unroll
+            for (int q = 0; q < 9; ++q) a.pos_fin[size_t(beg + t) * 9 + q] = T[q];
+            a.id_fin[beg + t] = a.id_in[beg + t];
+            ex.take(T, worst, rad2);
+        }
+        post();
         if (lane == 0) {
             nd->flags = 1u;
             nd->icount = 0;
@@ -375,12 +506,9 @@ __device__ __forceinline__ void level_node(const LevelArgs& a, uint32_t ni, uint
     // ---- split (OBBtree.cpp:43-108): the longest axis whose centre
     // projection leaves both sides non-empty, else index halves; the three
     // candidates are counted in one scan ----
-    AxisCand cand[3] = {{vlength(box.u), normalize(box.u)}, {vlength(box.v), normalize(box.v)},
-                        {vlength(box.w), normalize(box.w)}};
-    sort3_desc(cand);
+    AxisCand cand[3];
     float cp[3];
-#pragma unroll
-    for (int ch = 0; ch < 3; ++ch) cp[ch] = dot(box.c, cand[ch].dir);
+    split_candidates(box, cand, cp);
     uint32_t cnt[3] = {0, 0, 0};
     for (uint32_t c0 = 0; c0 < n; c0 += 64u * GROUP) {
         float T[GROUP][9];
@@ -388,15 +516,14 @@ __device__ __forceinline__ void level_node(const LevelArgs& a, uint32_t ni, uint
 #pragma unroll
         for (int j = 0; j < GROUP; ++j) {
             const bool valid = c0 + 64u * j + uint32_t(lane) < n;
+            if (valid) ex.take(T[j], worst, rad2);
 #pragma unroll
             for (int ch = 0; ch < 3; ++ch)
                 cnt[ch] += uint32_t(__popcll(__ballot(valid && goes_left(T[j], cand[ch].dir, cp[ch]))));
         }
     }
-    int pick = -1;
-#pragma unroll
-    for (int ch = 2; ch >= 0; --ch)
-        if (cnt[ch] != 0 && cnt[ch] != n) pick = ch;
+    post();
+    const int pick = split_pick(cnt, n);
     const bool ok = pick >= 0;
     f3 axis = cand[0].dir;
     float cproj = 0.f;
@@ -438,34 +565,30 @@ __device__ __forceinline__ void level_node(const LevelArgs& a, uint32_t ni, uint
             runR += uint32_t(__popcll(mR));
         }
     }
-    if (lane == 0) {
-        const uint32_t slot = next_first + atomicAdd(next_count, 2u);
-        BNode* k0 = &a.nodes[slot];
-        BNode* k1 = &a.nodes[slot + 1];
-        k0->mesh = nd->mesh; k0->beg = beg;      k0->end = beg + nl; k0->level = nd->level + 1; k0->flags = 0;
-        k1->mesh = nd->mesh; k1->beg = beg + nl; k1->end = end;      k1->level = nd->level + 1; k1->flags = 0;
-        nd->kid[0] = slot;
-        nd->kid[1] = slot + 1;
-        nd->flags = 0;
-        atomicMax(&a.mesh_depth[nd->mesh], nd->level + 1);
-    }
+    if (lane == 0) append_kids(a, nd, nl, next_first, next_count);
 }
 
-// One level of the build: lv[0] = {first node, node count} of this level
-// (written by the previous level's launch or by the host); the launch
-// writes lv[1] = {first node, count} of the next, its count grown by two
-// per split.  A fixed grid strides over the level's nodes, so levels can be
+// One level of the build: lv[0] = {first node, node count, big nodes, tiles}
+// of this level (written by the previous level's launches or by the host);
+// the launch writes lv[1] = {first node, count, ..} of the next, its count
+// grown by two per split.  A fixed grid strides over the level's nodes, so levels can be
 // launched back to back before their sizes are known on the host.
-__global__ __launch_bounds__(64) void k_level(LevelArgs a, uint2* lv) {
+__global__ __launch_bounds__(64) void k_level(LevelArgs a, uint4* lv) {
     __shared__ LevelShared S;
     const uint32_t first = lv[0].x, count = lv[0].y;
     const uint32_t next_first = first + count;
     if (blockIdx.x == 0 && threadIdx.x == 0) lv[1].x = next_first;
     for (uint32_t b = blockIdx.x; b < count; b += gridDim.x) {
+        const BNode& nd = a.nodes[first + b];
+        if (nd.end - nd.beg > a.big_min) continue;
         level_node(a, first + b, next_first, &lv[1].y, S);
         wave_sync();  // the next node reuses the LDS
     }
 }
+
+}  // namespace cdk
+#include "bigbuild.hpp"
+namespace cdk {
 
 // Left child = larger surface (OBBtree.cpp:101-107).
 __global__ void k_order_kids(BNode* nodes, uint32_t count) {
@@ -583,86 +706,6 @@ __global__ void k_emit_tris(const BNode* nodes, uint32_t count, const uint32_t* 
     }
 }
 
-// Containment slack of every box over its own triangles, and the mesh radius.
-__global__ __launch_bounds__(64) void k_slack(const BNode* nodes, uint32_t count, const float* pos_fin,
-                                              unsigned int* mesh_slack_bits, unsigned int* mesh_radius_bits) {
-    const uint32_t ni = blockIdx.x;
-    if (ni >= count) return;
-    const BNode& nd = nodes[ni];
-    const int lane = threadIdx.x;
-    const double u[3] = {nd.box[3], nd.box[4], nd.box[5]};
-    const double v[3] = {nd.box[6], nd.box[7], nd.box[8]};
-    const double w[3] = {nd.box[9], nd.box[10], nd.box[11]};
-    // a point's coordinates in the side vectors: its offset dotted with the
-    // dual basis (v x w, w x u, u x v) / det(u, v, w)
-    auto cross = [](const double* a, const double* b, double* o) {
-        o[0] = a[1] * b[2] - a[2] * b[1];
-        o[1] = a[2] * b[0] - a[0] * b[2];
-        o[2] = a[0] * b[1] - a[1] * b[0];
-    };
-    double du[3], dv[3], dw[3];
-    cross(v, w, du);
-    cross(w, u, dv);
-    cross(u, v, dw);
-    const double D = u[0] * du[0] + u[1] * du[1] + u[2] * du[2];
-    for (int k = 0; k < 3; ++k) {
-        du[k] = du[k] / D;
-        dv[k] = dv[k] / D;
-        dw[k] = dw[k] / D;
-    }
-    const double lu = sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
-    const double lv = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-    const double lw = sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
-    double worst = 0.0, rad = 0.0;
-    const uint32_t npts = 3 * (nd.end - nd.beg);
-    const float* P = pos_fin + size_t(nd.beg) * 9;
-    const double c[3] = {nd.box[0], nd.box[1], nd.box[2]};
-    const bool root = nd.level == 0;
-    for (uint32_t k0 = 0; k0 < npts; k0 += 64u * GROUP) {
-        float px[GROUP], py[GROUP], pz[GROUP];
-#pragma unroll
-        for (int j = 0; j < GROUP; ++j) {
-            const size_t k = min(k0 + 64u * j + uint32_t(lane), npts - 1);
-            px[j] = P[3 * k];
-            py[j] = P[3 * k + 1];
-            pz[j] = P[3 * k + 2];
-        }
-#pragma unroll
-        for (int j = 0; j < GROUP; ++j) {
-            if (k0 + 64u * j + uint32_t(lane) >= npts) continue;
-            const double p[3] = {px[j], py[j], pz[j]};
-            const double r[3] = {p[0] - c[0], p[1] - c[1], p[2] - c[2]};
-            double ex;
-            if (fabs(D) > 0.0) {
-                const double al = r[0] * du[0] + r[1] * du[1] + r[2] * du[2];
-                const double be = r[0] * dv[0] + r[1] * dv[1] + r[2] * dv[2];
-                const double ga = r[0] * dw[0] + r[1] * dw[1] + r[2] * dw[2];
-                ex = fmax(0.0, fabs(al) - 1.0) * lu + fmax(0.0, fabs(be) - 1.0) * lv + fmax(0.0, fabs(ga) - 1.0) * lw;
-            } else {
-                ex = INFINITY;
-            }
-            worst = fmax(worst, ex);
-            if (root) rad = fmax(rad, p[0] * p[0] + p[1] * p[1] + p[2] * p[2]);  // squared; roots only
-        }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        worst = fmax(worst, __shfl_xor(worst, off, 64));
-        rad = fmax(rad, __shfl_xor(rad, off, 64));
-    }
-    rad = sqrt(rad);  // sqrt is monotone: the root of the largest square is the largest root
-    if (lane == 0) {
-        // round up to float so the bound stays an upper bound
-        float wf = float(worst);
-        if (double(wf) < worst) wf = nextafterf(wf, INFINITY);
-        float rf = float(rad);
-        if (double(rf) < rad) rf = nextafterf(rf, INFINITY);
-        // one of SLACK_REPS copies per mesh, so a mesh's many nodes do not queue on one address
-        atomicMax(&mesh_slack_bits[size_t(nd.mesh) * SLACK_REPS + (ni % SLACK_REPS)], __float_as_uint(wf));
-        if (nd.level == 0) atomicMax(&mesh_radius_bits[nd.mesh], __float_as_uint(rf));
-    }
-}
-
 #define CK(x)                                                        \
     do {                                                             \
         hipError_t e_ = (x);                                         \
@@ -698,6 +741,9 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
     DevBuf* const ids = W + 2;  // ids[0], ids[1]
     DevBuf &pos_fin = W[4], &id_fin = W[5], &nodes = W[6], &mesh_depth = W[7], &level_tab = W[8], &base_nodes = W[9],
            &base_tris = W[10], &slack_bits = W[11], &radius_bits = W[12], &level_list = W[13];
+    DevBuf* const big_list = W + 14;   // big nodes of a level and the next
+    DevBuf* const tile_list = W + 16;  // their tiles
+    DevBuf &big_state = W[18], &tile_sums = W[19], &tile_ext = W[20], &tile_cnt = W[21], &tile_fn = W[22];
     std::vector<BNode> roots(nmesh);
     std::vector<std::pair<uint32_t, uint32_t>> levels;
     std::vector<uint32_t> host_ids;
@@ -705,6 +751,18 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
         radius(nmesh);
     uint64_t total_internal = 0;
     uint32_t first = 0, count = nmesh, cur = 0;
+    // the roots that take the tiled passes; every level's big nodes are
+    // disjoint, so their number and their tiles are bounded once
+    const uint32_t big_min = std::max(BIG_TRIS, ctx->leaf_max);
+    std::vector<BigNode> bigs;
+    std::vector<uint2> tiles;
+    for (uint32_t m = 0; m < nmesh; ++m) {
+        if (counts[m] <= big_min) continue;
+        for (uint32_t k = 0; k < big_tiles(counts[m]); ++k) tiles.push_back(make_uint2(uint32_t(bigs.size()), k));
+        bigs.push_back({m, uint32_t(tri_begin[m]), counts[m], uint32_t(tiles.size()) - big_tiles(counts[m])});
+    }
+    uint32_t nbig = uint32_t(bigs.size()), ntiles = uint32_t(tiles.size());
+    const size_t big_cap = size_t(T / big_min) + 1, tile_cap = size_t(T / TILE_TRIS) + big_cap;
     const size_t posb = std::max<uint64_t>(T, 1) * 9 * sizeof(float), idb = std::max<uint64_t>(T, 1) * sizeof(uint32_t);
 
     CK(pos[0].ensure(posb));
@@ -717,7 +775,20 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
     CK(mesh_depth.ensure(nmesh * sizeof(uint32_t)));
     CK(slack_bits.ensure(size_t(nmesh) * SLACK_REPS * sizeof(uint32_t)));
     CK(radius_bits.ensure(nmesh * sizeof(uint32_t)));
-    CK(level_tab.ensure((LEVEL_BATCH + 1) * sizeof(uint2)));
+    CK(level_tab.ensure((LEVEL_BATCH + 1) * sizeof(uint4)));
+    if (!bigs.empty()) {
+        CK(big_state.ensure(big_cap * sizeof(BigState)));
+        CK(tile_sums.ensure(tile_cap * sizeof(TileSums)));
+        CK(tile_ext.ensure(tile_cap * sizeof(TileExtents)));
+        CK(tile_cnt.ensure(tile_cap * sizeof(uint4)));
+        CK(tile_fn.ensure(tile_cap * 6 * 128 * sizeof(double2)));
+        for (int k = 0; k < 2; ++k) {
+            CK(big_list[k].ensure(big_cap * sizeof(BigNode)));
+            CK(tile_list[k].ensure(tile_cap * sizeof(uint2)));
+        }
+        CK(hipMemcpyAsync(big_list[0].p, bigs.data(), bigs.size() * sizeof(BigNode), hipMemcpyHostToDevice, st));
+        CK(hipMemcpyAsync(tile_list[0].p, tiles.data(), tiles.size() * sizeof(uint2), hipMemcpyHostToDevice, st));
+    }
     CK(base_nodes.ensure(nmesh * sizeof(uint32_t)));
     CK(base_tris.ensure(nmesh * sizeof(uint32_t)));
 
@@ -747,9 +818,10 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
     // launch takes its node range from the level table the previous one
     // filled, over a grid sized by an upper bound (a level at most doubles).
     while (count > 0) {
-        std::vector<uint2> tab(LEVEL_BATCH + 1, make_uint2(0u, 0u));
-        tab[0] = make_uint2(first, count);
-        CK(hipMemcpyAsync(level_tab.p, tab.data(), tab.size() * sizeof(uint2), hipMemcpyHostToDevice, st));
+        std::vector<uint4> tab(LEVEL_BATCH + 1, make_uint4(0u, 0u, 0u, 0u));
+        tab[0] = make_uint4(first, count, nbig, ntiles);
+        CK(hipMemcpyAsync(level_tab.p, tab.data(), tab.size() * sizeof(uint4), hipMemcpyHostToDevice, st));
+        uint64_t big_bound = nbig;
         uint64_t bound = count;
         for (uint32_t j = 0; j < LEVEL_BATCH; ++j) {
             LevelArgs a;
@@ -761,18 +833,51 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
             a.pos_fin = pos_fin.as<float>();
             a.id_fin = id_fin.as<uint32_t>();
             a.mesh_depth = mesh_depth.as<unsigned int>();
+            a.slack_bits = slack_bits.as<unsigned int>();
+            a.radius_bits = radius_bits.as<unsigned int>();
             a.leaf_max = ctx->leaf_max;
+            a.big_min = big_min;
+            uint4* const lv = level_tab.as<uint4>() + j;
+            if (big_bound) {
+                BigArgs b;
+                b.lv = a;
+                b.big = big_list[cur].as<BigNode>();
+                b.tiles = tile_list[cur].as<uint2>();
+                b.big_out = big_list[cur ^ 1].as<BigNode>();
+                b.tiles_out = tile_list[cur ^ 1].as<uint2>();
+                b.state = big_state.as<BigState>();
+                b.sums = tile_sums.as<TileSums>();
+                b.ext = tile_ext.as<TileExtents>();
+                b.counts = tile_cnt.as<uint4>();
+                b.fn = tile_fn.as<double2>();
+                b.tile_cap = uint32_t(tile_cap);
+                // big nodes at most double per level; a tile list holds at most tile_cap entries
+                const uint32_t gn = uint32_t(std::min<uint64_t>(big_bound, big_cap));
+                const uint32_t gt = uint32_t(std::min<uint64_t>(ntiles + big_bound, tile_cap));
+                hipLaunchKernelGGL(k_big_sums, dim3(gt), dim3(256), 0, st, b, lv);
+                hipLaunchKernelGGL(k_big_sim<3>, dim3(gt), dim3(192), 0, st, b, lv);
+                hipLaunchKernelGGL(k_big_resolve<3>, dim3(3 * gn), dim3(64 * (1 + RESOLVE_TILES)), 0, st, b, lv);
+                hipLaunchKernelGGL(k_big_sim<6>, dim3(gt), dim3(384), 0, st, b, lv);
+                hipLaunchKernelGGL(k_big_resolve<6>, dim3(6 * gn), dim3(64 * (1 + RESOLVE_TILES)), 0, st, b, lv);
+                hipLaunchKernelGGL(k_big_project, dim3(gt), dim3(256), 0, st, b, lv);
+                hipLaunchKernelGGL(k_big_count, dim3(gt), dim3(256), 0, st, b, lv);
+                hipLaunchKernelGGL(k_big_scatter, dim3(gt), dim3(256), 0, st, b, lv);
+                CK(hipGetLastError());
+                big_bound *= 2;
+            }
             const uint32_t grid = uint32_t(std::min<uint64_t>(bound, LEVEL_GRID));
-            hipLaunchKernelGGL(k_level, dim3(grid), dim3(64), 0, st, a, level_tab.as<uint2>() + j);
+            hipLaunchKernelGGL(k_level, dim3(grid), dim3(64), 0, st, a, lv);
             CK(hipGetLastError());
             cur ^= 1;
             bound = std::min<uint64_t>(2 * bound, node_cap);
         }
-        CK(hipMemcpyAsync(tab.data(), level_tab.p, tab.size() * sizeof(uint2), hipMemcpyDeviceToHost, st));
+        CK(hipMemcpyAsync(tab.data(), level_tab.p, tab.size() * sizeof(uint4), hipMemcpyDeviceToHost, st));
         CK(hipStreamSynchronize(st));
         for (uint32_t j = 0; j < LEVEL_BATCH && tab[j].y > 0; ++j) levels.push_back({tab[j].x, tab[j].y});
         first = tab[LEVEL_BATCH].x;
         count = tab[LEVEL_BATCH].y;
+        nbig = tab[LEVEL_BATCH].z;
+        ntiles = tab[LEVEL_BATCH].w;
     }
     {
         const uint32_t total = first;
@@ -842,9 +947,6 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
         hipLaunchKernelGGL(k_emit_tris, dim3(blocks_for(total, 256)), dim3(256), 0, st, nodes.as<BNode>(), total,
                            base_tris.as<uint32_t>(), pos_fin.as<float>(), id_fin.as<uint32_t>(), ctx->d_tris.as<float>(),
                            ctx->d_perm.as<uint32_t>(), ctx->d_leafof.as<uint32_t>());
-        CK(hipGetLastError());
-        hipLaunchKernelGGL(k_slack, dim3(total), dim3(64), 0, st, nodes.as<BNode>(), total, pos_fin.as<float>(),
-                           slack_bits.as<unsigned int>(), radius_bits.as<unsigned int>());
         CK(hipGetLastError());
         CK(hipMemcpyAsync(slack.data(), slack_bits.p, size_t(nmesh) * SLACK_REPS * sizeof(uint32_t),
                           hipMemcpyDeviceToHost, st));

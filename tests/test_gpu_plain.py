@@ -67,6 +67,41 @@ def test_tree_build_matches_oracle(gpu, gpu_l1, orc, L):
         assert np.array_equal(got["perm"], want["perm"]), name
 
 
+def _tiled_mesh(kind, n):
+    """n triangles whose coordinate sums are of one kind: order of magnitude
+    changes, half-way roundings and zeros of a running double sum."""
+    rng = np.random.default_rng(1000 + n)
+    if kind == "grid":  # rows that swing through zero; one axis all zeros
+        k = np.arange(3 * n)
+        return np.stack([(k % 97) - 48.0, np.zeros(3 * n), (k // 97) * 0.5], 1).astype(np.float32).reshape(n, 9)
+    if kind == "offset":  # far from the origin: large sums, cancelling moments
+        return (rng.normal(size=(n, 9)) + 3000.0).astype(np.float32)
+    if kind == "dyadic":  # few bits over many binades: half-way cases
+        m = rng.integers(-8, 9, size=(n, 9)) * np.exp2(rng.integers(-30, 30, size=(n, 9)))
+        return m.astype(np.float32)
+    if kind == "same":  # one distinct point: no box
+        return np.full((n, 9), 2.5, np.float32)
+    return (rng.normal(size=(n, 9)) * np.exp(rng.normal(size=(n, 1)) * 3.0)).astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", ["grid", "offset", "dyadic", "same", "spread"])
+def test_tree_build_tiled_nodes(gpu, orc, kind):
+    """Nodes above the tiled passes' threshold (1,024 triangles, tiles of 512,
+    chunks of 8), around each edge and several in one batch: bit-identical to
+    the oracle's sequential sums, and the slack covers the oracle's."""
+    sizes = [1024, 1025, 1031, 1536, 1537, 2048, 2049, 3333] + ([] if kind == "same" else [20011])
+    meshes = [_tiled_mesh(kind, n) for n in sizes]
+    case(f"tiled tree build {kind} sizes={sizes}")
+    for n, m, mid in zip(sizes, meshes, gpu.register_soups(meshes)):
+        tree = orc.tree(m, 4)
+        want, got = tree.export(), gpu.export_tree(mid)
+        assert got["root"].tobytes() == want["root"].tobytes(), n
+        assert got["obbs"].tobytes() == want["obbs"].tobytes(), n
+        assert np.array_equal(got["links"], want["links"]), n
+        assert np.array_equal(got["perm"], want["perm"]), n
+        assert gpu.mesh_info(mid)["slack"] >= np.float32(tree.slack) * (1 - 1e-6), n
+
+
 def test_tree_build_hand_derived_splits(gpu_l1, orc):
     """The split cases derived by hand (tie to the left, an axis that leaves a
     side empty, index halves, the larger-surface swap): the GPU build gives
