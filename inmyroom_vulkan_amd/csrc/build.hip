@@ -315,11 +315,9 @@ __device__ inline void post_excess(const LevelArgs& a, const BNode& nd, uint32_t
     if (nd.level == 0) atomicMax(&a.radius_bits[nd.mesh], __float_as_uint(round_up(sqrt(rad2))));
 }
 
-// The children of a split node, appended to the next level.
-__device__ inline uint32_t append_kids(const LevelArgs& a, BNode* nd, uint32_t nl, uint32_t next_first,
-                                       unsigned int* next_count) {
+// The children of a split node, in the next level's slots `slot` and slot + 1.
+__device__ inline void place_kids(const LevelArgs& a, BNode* nd, uint32_t nl, uint32_t slot) {
     const uint32_t beg = nd->beg, end = nd->end;
-    const uint32_t slot = next_first + atomicAdd(next_count, 2u);
     BNode* k0 = &a.nodes[slot];
     BNode* k1 = &a.nodes[slot + 1];
     k0->mesh = nd->mesh; k0->beg = beg;      k0->end = beg + nl; k0->level = nd->level + 1; k0->flags = 0;
@@ -327,6 +325,12 @@ __device__ inline uint32_t append_kids(const LevelArgs& a, BNode* nd, uint32_t n
     nd->kid[0] = slot;
     nd->kid[1] = slot + 1;
     nd->flags = 0;
+}
+// The same, taking the next two free slots of the level.
+__device__ inline uint32_t append_kids(const LevelArgs& a, BNode* nd, uint32_t nl, uint32_t next_first,
+                                       unsigned int* next_count) {
+    const uint32_t slot = next_first + atomicAdd(next_count, 2u);
+    place_kids(a, nd, nl, slot);
     atomicMax(&a.mesh_depth[nd->mesh], nd->level + 1);
     return slot;
 }
@@ -568,6 +572,178 @@ __device__ __forceinline__ void level_node(const LevelArgs& a, uint32_t ni, uint
     if (lane == 0) append_kids(a, nd, nl, next_first, next_count);
 }
 
+// Nodes of few triangles, one lane each: the deepest levels hold most of the
+// nodes, and a wavefront per node of a few triangles leaves most lanes idle
+// and runs eig3 on one of them.  Each lane runs the reference's loops as they
+// are written.
+constexpr uint32_t TINY_TRIS = 16;
+
+// One triangle's coordinates at a time, TINY_FETCH in flight (indices clamped, as above).
+constexpr uint32_t TINY_FETCH = 3;
+template <class F>
+__device__ __forceinline__ void tiny_tris(const float* __restrict__ P, uint32_t n, F f) {
+    for (uint32_t i0 = 0; i0 < n; i0 += TINY_FETCH) {
+        float T[TINY_FETCH][9];
+#pragma unroll
+        for (uint32_t j = 0; j < TINY_FETCH; ++j) {
+            const float* p = P + 9 * size_t(min(i0 + j, n - 1));
+#pragma unroll
+            for (int q = 0; q < 9; ++q) T[j][q] = p[q];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < TINY_FETCH; ++j)
+            if (i0 + j < n) f(i0 + j, T[j]);
+    }
+}
+
+__global__ __launch_bounds__(64) void k_level_tiny(LevelArgs a, uint4* lv) {
+    const uint32_t first = lv[0].x, count = lv[0].y, next_first = first + count;
+    const uint32_t lane = threadIdx.x;
+    for (uint32_t b0 = blockIdx.x * 64u; b0 < count; b0 += gridDim.x * 64u) {
+        const uint32_t ni = first + b0 + lane;
+        BNode* nd = nullptr;
+        uint32_t beg = 0, n = 0;
+        if (b0 + lane < count) {
+            nd = &a.nodes[ni];
+            beg = nd->beg;
+            n = nd->end - beg;
+            if (n > TINY_TRIS || n == 0) nd = nullptr;  // the other passes' (an empty mesh's root is the wavefronts')
+        }
+        if (!nd) n = 0;
+        const float* P = a.pos_in + size_t(beg) * 9;
+        double worst = 0.0, rad2 = 0.0;
+        uint32_t nl = 0;
+        bool splits = false;
+        if (nd) {
+            bool multi = false;
+            double m[3] = {0.0, 0.0, 0.0};
+            const float x0 = P[0], y0 = P[1], z0 = P[2];
+            tiny_tris(P, n, [&](uint32_t, const float (&T)[9]) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    multi |= !(T[3 * k] == x0 && T[3 * k + 1] == y0 && T[3 * k + 2] == z0);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) m[q] = m[q] + double(T[3 * k + q]);
+                }
+            });
+            Box box = empty_box(mk(x0, y0, z0));
+            if (multi) {
+                const double N = double(3 * n);
+                m[0] = m[0] / N;
+                m[1] = m[1] / N;
+                m[2] = m[2] / N;
+                double c[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};  // xx, yy, zz, xy, xz, yz (OBB.cpp:56-73)
+                tiny_tris(P, n, [&](uint32_t, const float (&T)[9]) {
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        const double dx = double(T[3 * k]) - m[0], dy = double(T[3 * k + 1]) - m[1],
+                                     dz = double(T[3 * k + 2]) - m[2];
+                        c[0] = c[0] + dx * dx;
+                        c[1] = c[1] + dy * dy;
+                        c[2] = c[2] + dz * dz;
+                        c[3] = c[3] + dx * dy;
+                        c[4] = c[4] + dx * dz;
+                        c[5] = c[5] + dy * dz;
+                    }
+                });
+#pragma unroll
+                for (int k = 0; k < 6; ++k) c[k] = c[k] / N;
+                double A[3][3] = {{c[0], c[3], c[4]}, {c[3], c[1], c[5]}, {c[4], c[5], c[2]}};
+                double V[3][3], d[3], ax[9];
+                eig3(A, V, d);
+                for (int r = 0; r < 3; ++r)
+                    for (int q = 0; q < 3; ++q) ax[r * 3 + q] = V[r][q];
+                double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+                tiny_tris(P, n, [&](uint32_t, const float (&T)[9]) {
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) {
+                            const double pr = (ax[3 * q] * double(T[3 * k]) + ax[3 * q + 1] * double(T[3 * k + 1])) +
+                                              ax[3 * q + 2] * double(T[3 * k + 2]);
+                            if (!(lo[q] < pr)) lo[q] = pr;
+                            if (hi[q] < pr) hi[q] = pr;
+                        }
+                });
+                float bx[12];
+                box_of_extents(ax, lo, hi, bx);
+                box = box_from12(bx);
+            }
+            box_to12(box, nd->box);
+            nd->surf = surface(box);
+            const Excess ex(box);
+            if (n <= a.leaf_max) {
+                tiny_tris(P, n, [&](uint32_t i, const float (&T)[9]) {
+                    ex.take(T, worst, rad2);
+                    float* o = a.pos_fin + size_t(beg + i) * 9;
+#pragma unroll
+                    for (int q = 0; q < 9; ++q) o[q] = T[q];
+                    a.id_fin[beg + i] = a.id_in[beg + i];
+                });
+                nd->flags = 1u;
+                nd->icount = 0;
+                nd->tcount = n;
+            } else {
+                splits = true;
+                AxisCand cand[3];
+                float cp[3];
+                split_candidates(box, cand, cp);
+                uint32_t cnt[3] = {0, 0, 0};
+                tiny_tris(P, n, [&](uint32_t, const float (&T)[9]) {
+                    ex.take(T, worst, rad2);
+#pragma unroll
+                    for (int ch = 0; ch < 3; ++ch) cnt[ch] += goes_left(T, cand[ch].dir, cp[ch]) ? 1u : 0u;
+                });
+                const int pick = split_pick(cnt, n);
+                f3 axis = cand[0].dir;
+                float cproj = 0.f;
+                nl = n / 2;
+#pragma unroll
+                for (int ch = 0; ch < 3; ++ch)
+                    if (ch == pick) {
+                        axis = cand[ch].dir;
+                        cproj = cp[ch];
+                        nl = cnt[ch];
+                    }
+                uint32_t l = beg, r = beg + nl;
+                tiny_tris(P, n, [&](uint32_t i, const float (&T)[9]) {
+                    const bool left = pick >= 0 ? goes_left(T, axis, cproj) : i < n / 2;
+                    const uint32_t dst = left ? l++ : r++;
+                    float* o = a.pos_out + size_t(dst) * 9;
+#pragma unroll
+                    for (int q = 0; q < 9; ++q) o[q] = T[q];
+                    a.id_out[dst] = a.id_in[beg + i];
+                });
+            }
+        }
+        // the wavefront's children take one atomic, and so do its excesses
+        // when its nodes are one mesh's below the root
+        const unsigned long long live = __ballot(nd != nullptr), kids = __ballot(splits);
+        if (!live) continue;
+        uint32_t slot = 0;
+        if (kids) {
+            if (lane == 0) slot = atomicAdd(&lv[1].y, 2u * uint32_t(__popcll(kids)));
+            slot = uint32_t(__builtin_amdgcn_readfirstlane(int(slot)));
+            slot += next_first + 2u * uint32_t(__popcll(kids & (lane == 0 ? 0ull : (~0ull >> (64 - lane)))));
+            if (splits) place_kids(a, nd, nl, slot);
+        }
+        const int src = __builtin_ctzll(live);
+        const uint32_t mesh = nd ? nd->mesh : 0u, level = nd ? nd->level : 0u;
+        const uint32_t mesh0 = uint32_t(__shfl(int(mesh), src, 64)), level0 = uint32_t(__shfl(int(level), src, 64));
+        if (level0 > 0 && __ballot(nd && mesh != mesh0) == 0) {
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) worst = fmax(worst, __shfl_xor(worst, off, 64));
+            if (int(lane) == src) {
+                post_excess(a, *nd, ni, worst, rad2);
+                if (kids) atomicMax(&a.mesh_depth[mesh], level + 1);
+            }
+        } else if (nd) {
+            post_excess(a, *nd, ni, worst, rad2);
+            if (splits) atomicMax(&a.mesh_depth[mesh], level + 1);
+        }
+    }
+}
+
 // One level of the build: lv[0] = {first node, node count, big nodes, tiles}
 // of this level (written by the previous level's launches or by the host);
 // the launch writes lv[1] = {first node, count, ..} of the next, its count
@@ -580,7 +756,8 @@ __global__ __launch_bounds__(64) void k_level(LevelArgs a, uint4* lv) {
     if (blockIdx.x == 0 && threadIdx.x == 0) lv[1].x = next_first;
     for (uint32_t b = blockIdx.x; b < count; b += gridDim.x) {
         const BNode& nd = a.nodes[first + b];
-        if (nd.end - nd.beg > a.big_min) continue;
+        const uint32_t n = nd.end - nd.beg;
+        if (n > a.big_min || (n <= TINY_TRIS && n > 0)) continue;
         level_node(a, first + b, next_first, &lv[1].y, S);
         wave_sync();  // the next node reuses the LDS
     }
@@ -718,7 +895,7 @@ __global__ void k_emit_tris(const BNode* nodes, uint32_t count, const uint32_t* 
 static inline uint32_t blocks_for(uint64_t n, uint32_t b) { return uint32_t((n + b - 1) / b); }
 
 constexpr uint32_t LEVEL_BATCH = 8;     // level launches per wait of the build
-constexpr uint32_t LEVEL_GRID = 65536;  // workgroups of a level launch at most (larger levels are strided)
+constexpr uint32_t LEVEL_GRID = 8192;  // workgroups of a level launch at most (larger levels are strided)
 
 // Build every soup of the batch and append the trees to the context arenas.
 BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, uint32_t nmesh, bool tri9_on_device) {
@@ -867,6 +1044,8 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
             }
             const uint32_t grid = uint32_t(std::min<uint64_t>(bound, LEVEL_GRID));
             hipLaunchKernelGGL(k_level, dim3(grid), dim3(64), 0, st, a, lv);
+            const uint32_t tiny_grid = std::min<uint32_t>(blocks_for(bound, 64), LEVEL_GRID);
+            hipLaunchKernelGGL(k_level_tiny, dim3(tiny_grid), dim3(64), 0, st, a, lv);
             CK(hipGetLastError());
             cur ^= 1;
             bound = std::min<uint64_t>(2 * bound, node_cap);
