@@ -1720,7 +1720,7 @@ int ensure_step(cd_ctx* ctx, const StepArgs& a, uint64_t* fcap) {
         HCK(ctx, ctx->d_work[W_SHOTS].ensure(size_t(R) * sizeof(RayShot)));
         HCK(ctx, ctx->d_work[W_RESP].ensure(size_t(P) * sizeof(cd_pair_response)));
         if (a.stack_entries > uint32_t(RAY_STACK_ENTRIES)) {  // trees deeper than the LDS stack holds
-            const size_t blocks = (2 * size_t(R) + 63) / 64;
+            const size_t blocks = shoot_blocks(uint32_t(R));
             HCK(ctx, ctx->d_work[W_GSTACK].ensure(blocks * 2 * a.stack_entries * 64 * sizeof(uint32_t)));
         }
     }
@@ -2098,7 +2098,7 @@ int cd_shoot_rays(cd_ctx* ctx, const cd_shoot_params* params, cd_pair_response* 
     const uint32_t* pbegin = ctx->d_work[W_PIDS].as<uint32_t>() + 2 * size_t(nq);
     uint32_t* gstack = nullptr;  // trees deeper than the LDS stack holds: the stacks in HBM
     if (stack_entries > uint32_t(RAY_STACK_ENTRIES)) {
-        const size_t blocks = (2 * ctx->ray_total + 63) / 64;
+        const size_t blocks = shoot_blocks(uint32_t(ctx->ray_total));
         HCK(ctx, ctx->d_work[W_GSTACK].ensure(blocks * 2 * stack_entries * 64 * sizeof(uint32_t)));
         gstack = ctx->d_work[W_GSTACK].as<uint32_t>();
     }

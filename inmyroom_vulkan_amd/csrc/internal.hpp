@@ -98,16 +98,17 @@ struct RayShot {
     uint32_t ok;    // bit p: pass p succeeded
     uint32_t pair;  // query (entity pair) of the ray
 };
-// The box-only terms of the ray shooting's box test for one stored box
-// (centre c, half-sides u, v, w): the three slab normals v x w, w x u, u x v,
-// the box's projection radius on each, and the 1-norm sums of c and of
-// u, v, w that bound the test's rounding.  Computed once per box (after each
-// build or refit of its mesh) with the very operations the test would use.
+// What the ray shooting's walk reads of one stored box (centre c, half-sides
+// u, v, w): the three slab normals v x w, w x u, u x v, the box's projection
+// radius on each, the centre, and the child as a stack entry.  Computed once
+// per box (after each build or refit of its mesh); 128 bytes a node where its
+// child records, and these terms beside them, took 256: over meshes that L2
+// does not hold the walk waits on those lines.
 struct alignas(64) RaySlab {
     float n[9];
     float h[3];
-    float cr, sr;
-    float pad[2];
+    float c[3];
+    uint32_t entry;  // link | leaf triangles (0: an internal node) << RAY_LINK_BITS
 };
 static_assert(sizeof(RaySlab) == 64, "slab record layout");
 

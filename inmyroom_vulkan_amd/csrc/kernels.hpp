@@ -108,7 +108,7 @@ hipError_t launch_sort_perm(const cd_contact* in, uint32_t n, int f_hi, int f_mi
 // response.hip
 // pbegin: per side (nq each) the first ray of every pair, non-decreasing;
 // stack_entries: the deepest tree the rays meet + 2; above RAY_STACK_ENTRIES
-// the stacks live in gstack, ceil(2 nrays / 64) * 2 * stack_entries * 64
+// the stacks live in gstack, shoot_blocks(nrays) * 2 * stack_entries * 64
 // words; ctr->err gets bit 0 if a traversal stack would have overflowed,
 // ctr->sat the boxes tested and ctr->tritests the ray-triangle tests.
 // stride: the per-side spacing of pbegin (0: nq); dc: the step's count block
@@ -116,6 +116,7 @@ hipError_t launch_sort_perm(const cd_contact* in, uint32_t n, int f_hi, int f_mi
 // nq being the capacities.
 // slabs / roots: the slab records of every node's children and every mesh's
 // root (launch_ray_slabs), current for the meshes the rays meet.
+uint32_t shoot_blocks(uint32_t nrays);  // wavefronts of a launch over nrays rays
 hipError_t launch_shoot(const cd_ray* rays, uint32_t nrays, uint32_t base1, const uint32_t* pbegin, uint32_t nq,
                         const QueryRec* qs, const MeshRec* meshes, const NodeRec* nodes, const RaySlab* slabs,
                         const RaySlab* roots, const float* tris,

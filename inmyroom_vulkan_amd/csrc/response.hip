@@ -21,6 +21,8 @@
 // distance is not negative and, when it is popped, its entry distance is
 // below the best hit so far: the nodes visited, and the order in which equal
 // distances are met, are those of the reference's recursion.
+#include <algorithm>
+
 #include "rayattr.hpp"
 
 namespace cdk {
@@ -75,8 +77,9 @@ __device__ __forceinline__ bool ray_triangle(f3 dir, f3 v0, f3 v1, f3 v2, float&
 // transform and no normalised normal per test.
 struct LocalRay {
     f3 o, d;
-    float on, dn;   // |o|_1, |d|_1
+    float on;       // |o|_1
     float kappa;    // relative rounding margin of the box tests, grown with A's condition number
+    float dk;       // 4 kappa |d|_1
     bool ok;        // A invertible: else every box is entered
 };
 __device__ __forceinline__ float norm1f(f3 v) { return (fabsf(v.x) + fabsf(v.y)) + fabsf(v.z); }
@@ -90,14 +93,15 @@ __device__ __forceinline__ LocalRay local_ray(const M4& C, f3 dir) {
     L.o = mk(-dot(r0, c) * inv, -dot(r1, c) * inv, -dot(r2, c) * inv);
     L.d = mk(dot(r0, dir) * inv, dot(r1, dir) * inv, dot(r2, dir) * inv);
     L.on = norm1f(L.o);
-    L.dn = norm1f(L.d);
+    const float dn = norm1f(L.d);
     // |A|_F |A^-1|_F is 3 for a rotation times a uniform scale
     const float fa = sqrtf((dot(a0, a0) + dot(a1, a1)) + dot(a2, a2));
     const float fi = sqrtf((dot(r0, r0) + dot(r1, r1)) + dot(r2, r2)) * fabsf(inv);
     const float cond = fa * fi * (1.f / 3.f);
     L.kappa = 0x1p-16f * (cond > 1.f ? cond : 1.f);
+    L.dk = 4.f * L.kappa * dn;
     L.ok = det != 0.f && __builtin_isfinite(inv) && __builtin_isfinite(L.kappa) && L.kappa < 0x1p-4f &&
-           __builtin_isfinite(L.on) && __builtin_isfinite(L.dn);
+           __builtin_isfinite(L.on) && __builtin_isfinite(dn);
     return L;
 }
 // Ray::IntersectParalgram from the origin (Ray.cpp:36-133): the three slabs
@@ -135,22 +139,9 @@ __device__ __forceinline__ bool ray_box(f3 dir, const Box& b, float& tmin, float
     return true;
 }
 
-// The mesh-frame test of a stored box (centre c, half-sides u, v, w): the
-// three slabs of Ray::IntersectParalgram (Ray.cpp:36-133), normals v x w,
-// w x u, u x v, each slab's half-width the box's projection radius on its
-// normal.  Every slab and crossing parameter is computed once and bounded by
-// its rounding (kappa, and the relative error of the crossing's
-// denominator), giving a widened and a shrunk interval.  BOX_OUT: even the
-// widened interval misses, so the exact ray misses and so does the
-// reference's float test, whose rounding is far inside these bounds.
-// BOX_IN: even the shrunk interval meets the ray ahead of its origin.
-// BOX_NEAR: the decision is within rounding (a box the ray grazes, one ending
-// at the ray's origin, a flat box, a slab the ray runs along); the caller
-// then runs the reference's own test.  tmin/tmax: the unwidened parameters,
-// for the order of the children and the pruning against the best hit.
-// The box-only terms (RaySlab), computed once per stored box.
-__device__ __forceinline__ RaySlab make_slab(const float* bx) {
-    const f3 c = mk(bx[0], bx[1], bx[2]);
+// What a walk reads of a stored box (RaySlab), computed once per box.
+__device__ __forceinline__ RaySlab make_slab(const ChildRec& r) {
+    const float* bx = r.box;
     const f3 u = mk(bx[3], bx[4], bx[5]), v = mk(bx[6], bx[7], bx[8]), w = mk(bx[9], bx[10], bx[11]);
     const f3 nrm[3] = {cross(v, w), cross(w, u), cross(u, v)};
     RaySlab s;
@@ -161,60 +152,78 @@ __device__ __forceinline__ RaySlab make_slab(const float* bx) {
         s.n[3 * k + 1] = n.y;
         s.n[3 * k + 2] = n.z;
         s.h[k] = (fabsf(dot(n, u)) + fabsf(dot(n, v))) + fabsf(dot(n, w));
+        s.c[k] = bx[k];
     }
-    s.cr = norm1f(c);
-    s.sr = (norm1f(u) + norm1f(v)) + norm1f(w);
-    s.pad[0] = s.pad[1] = 0.f;
+    s.entry = r.link | (child_cnt(r) << RAY_LINK_BITS);
     return s;
 }
+
+// The mesh-frame test of a stored box (centre c, half-sides u, v, w): the
+// three slabs of Ray::IntersectParalgram (Ray.cpp:36-133), normals v x w,
+// w x u, u x v, each slab's half-width the box's projection radius on its
+// normal.  Every slab and crossing parameter is computed once and bounded by
+// its rounding (kappa, and the relative error rho of the crossing's
+// denominator), giving a widened and a shrunk interval.  BOX_OUT: even the
+// widened interval misses, so the exact ray misses and so does the
+// reference's float test, whose rounding is far inside these bounds.
+// BOX_IN: even the shrunk interval meets the ray ahead of its origin.
+// BOX_NEAR: the decision is within rounding (a box the ray grazes, one ending
+// at the ray's origin, a flat box, a slab the ray runs along); the caller
+// then runs the reference's own test.  tmin/tmax: the unwidened parameters,
+// for the order of the children and the pruning against the best hit.
+// The crossings of a slab widened by e lie e |r| further out, and rho of
+// their own size beyond that, so both intervals differ from the crossing t by
+// at most e |r| (1 + rho) + rho |t|.  e is bounded by the 1-norms of the
+// normal, the centre and the half-sides; the latter's from the record: the
+// sides are orthogonal, so |u|_1 <= sqrt(3) |u| <= 3 h / |n|_1.  Written without branches: a node's two
+// tests are most of a step's instructions, with about one wavefront per SIMD,
+// and the exec-mask turns of the branches cost as much as the arithmetic.
 enum : int { BOX_OUT = 0, BOX_IN = 1, BOX_NEAR = 2 };
-__device__ __forceinline__ int box_local(const LocalRay& R, const float* bx, const RaySlab& sl, float& tmin,
-                                         float& tmax) {
-    tmin = -__builtin_huge_valf();
-    tmax = __builtin_huge_valf();
-    if (!R.ok) return BOX_NEAR;
-    const f3 c = mk(bx[0], bx[1], bx[2]);
+__device__ __forceinline__ int box_local(const LocalRay& R, const RaySlab& sl, float& tmin, float& tmax) {
+    const float inf = __builtin_huge_valf();
+    tmin = -inf;
+    tmax = inf;
+    const f3 c = mk(sl.c[0], sl.c[1], sl.c[2]);
     const f3 q = sub(R.o, c);
-    const float reach = ((norm1f(q) + R.on) + sl.cr) + sl.sr;
-    const f3 nrm[3] = {mk(sl.n[0], sl.n[1], sl.n[2]), mk(sl.n[3], sl.n[4], sl.n[5]), mk(sl.n[6], sl.n[7], sl.n[8])};
-    float lo_w = -__builtin_huge_valf(), hi_w = __builtin_huge_valf();
-    float lo_s = -__builtin_huge_valf(), hi_s = __builtin_huge_valf();
+    float nn[3], sides = 0.f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        nn[k] = norm1f(mk(sl.n[3 * k], sl.n[3 * k + 1], sl.n[3 * k + 2]));
+        sides = __builtin_fmaf(sl.h[k], __builtin_amdgcn_rcpf(nn[k]), sides);
+    }
+    const float reach = __builtin_fmaf(3.1f, sides, (norm1f(q) + R.on) + norm1f(c));  // infinite or NaN without a normal
+    const float kr = R.kappa * reach;
+    float lo_w = -inf, hi_w = inf, lo_s = -inf, hi_s = inf;
     bool decided = true;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        const f3 n = nrm[k];
-        const float nn = norm1f(n);
+        const f3 n = mk(sl.n[3 * k], sl.n[3 * k + 1], sl.n[3 * k + 2]);
         const float h = sl.h[k];
-        const float e = R.kappa * nn * reach;  // bound on the rounding of h and num
+        const float e = kr * nn[k];     // bound on the rounding of h and num
+        const float d4 = R.dk * nn[k];  // four times the bound on den's rounding
         const float num = dot(n, q);
         const float den = dot(n, R.d);
-        const float dl = R.kappa * nn * R.dn;  // bound on den's rounding
-        if (fabsf(den) > 4.f * dl && fabsf(den) > 0x1p-100f) {
-            const float r = __builtin_amdgcn_rcpf(den);  // within an ulp, far inside rho
-            const float rho = 2.f * dl * fabsf(r) + R.kappa;  // relative error of a crossing parameter
-            const float sg = r < 0.f ? -1.f : 1.f;  // the crossing through -h is the entry when den > 0
-            const float t1 = (-h - num) * r, t2 = (h - num) * r;
-            tmin = max_std(sg > 0.f ? t1 : t2, tmin);
-            tmax = min_std(sg > 0.f ? t2 : t1, tmax);
-            const float w1 = (-(h + e) - num) * r, w2 = ((h + e) - num) * r;
-            const float a = sg > 0.f ? w1 : w2, b = sg > 0.f ? w2 : w1;
-            lo_w = max_std(a - rho * fabsf(a), lo_w);
-            hi_w = min_std(b + rho * fabsf(b), hi_w);
-            if (h > e) {
-                const float s1 = (-(h - e) - num) * r, s2 = ((h - e) - num) * r;
-                const float as = sg > 0.f ? s1 : s2, bs = sg > 0.f ? s2 : s1;
-                lo_s = max_std(as + rho * fabsf(as), lo_s);
-                hi_s = min_std(bs - rho * fabsf(bs), hi_s);
-            } else {
-                decided = false;  // a slab thinner than its rounding
-            }
-        } else if (!(fabsf(num) + e < h)) {
-            decided = false;  // runs along the slab, not clearly inside it
-        }
+        const bool cuts = fabsf(den) > fmaxf(d4, 0x1p-100f);  // else the ray runs along the slab
+        const float r = __builtin_amdgcn_rcpf(cuts ? den : 1.f);  // within an ulp, far inside rho
+        const float ar = fabsf(r);
+        const float rho = __builtin_fmaf(0.5f * d4, ar, R.kappa);  // relative error of a crossing parameter
+        const float t1 = (-h - num) * r, t2 = (h - num) * r;
+        const float a = fminf(t1, t2), b = fmaxf(t1, t2);
+        const float m0 = e * ar, m = __builtin_fmaf(rho, m0, m0);
+        const float ma = __builtin_fmaf(rho, fabsf(a), m), mb = __builtin_fmaf(rho, fabsf(b), m);
+        tmin = fmaxf(cuts ? a : -inf, tmin);
+        tmax = fminf(cuts ? b : inf, tmax);
+        lo_w = fmaxf(cuts ? a - ma : -inf, lo_w);
+        hi_w = fminf(cuts ? b + mb : inf, hi_w);
+        lo_s = fmaxf(cuts ? a + ma : -inf, lo_s);
+        hi_s = fminf(cuts ? b - mb : inf, hi_s);
+        // a slab thinner than its rounding, or one the ray runs along and is not clearly inside
+        decided &= cuts ? h > e : fabsf(num) + e < h;
     }
-    if (!(lo_w <= hi_w && hi_w >= 0.f)) return BOX_OUT;
-    if (decided && lo_s <= hi_s && hi_s >= 0.f) return BOX_IN;
-    return BOX_NEAR;
+    const bool usable = R.ok & (reach < 0x1p100f);
+    const bool out = !((lo_w <= hi_w) & (hi_w >= 0.f));
+    const bool in = decided & (lo_s <= hi_s) & (hi_s >= 0.f);
+    return !usable ? BOX_NEAR : out ? BOX_OUT : in ? BOX_IN : BOX_NEAR;
 }
 
 struct Hit {
@@ -222,41 +231,6 @@ struct Hit {
     float dist, bx, by;
     uint32_t tri;  // mesh-local tree-order slot
 };
-
-// A leaf's triangles are fetched LEAF_FETCH at a time (their loads overlap),
-// then tested in order.
-constexpr uint32_t LEAF_FETCH = 4;
-__device__ __forceinline__ void leaf_hits(const float* __restrict__ tris, const MeshRec& m, const M4& C, f3 dir, uint32_t off,
-                          uint32_t cnt, Hit& best) {
-    for (uint32_t i0 = off; i0 < off + cnt; i0 += LEAF_FETCH) {
-        const uint32_t k = min(LEAF_FETCH, off + cnt - i0);
-        float t9[LEAF_FETCH][9];
-#pragma unroll
-        for (uint32_t u = 0; u < LEAF_FETCH; ++u)
-            if (u < k) {
-                const float* src = tris + (size_t(m.tri_base) + i0 + u) * 9;
-#pragma unroll
-                for (int e = 0; e < 9; ++e) t9[u][e] = src[e];
-            }
-#pragma unroll
-        for (uint32_t u = 0; u < LEAF_FETCH; ++u) {
-            if (u >= k) break;
-            const f3 P0 = mul4(C, mk(t9[u][0], t9[u][1], t9[u][2]), 1.f);
-            const f3 P1 = mul4(C, mk(t9[u][3], t9[u][4], t9[u][5]), 1.f);
-            const f3 P2 = mul4(C, mk(t9[u][6], t9[u][7], t9[u][8]), 1.f);
-            float bx = 0.f, by = 0.f, dist = __builtin_huge_valf();
-            bool back = false;
-            if (ray_triangle(dir, P0, P1, P2, bx, by, dist, back) && dist > 0.f && dist < best.dist) {
-                best.hit = true;
-                best.back = back;
-                best.dist = dist;
-                best.tri = i0 + u;
-                best.bx = bx;
-                best.by = by;
-            }
-        }
-    }
-}
 
 // Per-lane traversal stack in LDS, entry-major (entry e of lane l at
 // e * 64 + l, so a wavefront's accesses fall in distinct banks).  An entry
@@ -272,8 +246,8 @@ struct RayStack {
     float* t0;
     int lane;
     int cap;  // entries per lane
-    __device__ __forceinline__ void put(int i, uint32_t l, uint32_t c, float t) {
-        lc[i * 64 + lane] = l | (c << RAY_LINK_BITS);
+    __device__ __forceinline__ void put(int i, uint32_t entry, float t) {
+        lc[i * 64 + lane] = entry;
         t0[i * 64 + lane] = t;
     }
 };
@@ -301,98 +275,262 @@ __device__ __forceinline__ float partner(float* sbest, int lane) {
 // is skipped, and the walk stops once the partner ends without a back-face
 // hit (the pass fails whatever this walk finds).
 constexpr float BOUND_SLACK = 1.f + 0x1p-12f;
-// nslab: the slab records of this mesh's nodes' children (2 per node),
-// rslab: its root's.
-__device__ __forceinline__ Hit ray_tree(const MeshRec& m, const NodeRec* __restrict__ nodes,
+
+// What a wavefront's walks share in LDS.
+struct WalkShared {
+    float best[64];     // the lanes' published best hits
+    float ray[15][64];  // each lane's walk: its mesh-to-ray matrix (columns' x, y, z) and direction
+    uint32_t tri[64], own[64];  // the leaf tests of a step: triangle, and the lane whose walk it belongs to
+};
+__device__ __forceinline__ void wave_order() { __builtin_amdgcn_wave_barrier(); }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_addu(uint32_t v) {
+    return v + uint32_t(__builtin_amdgcn_update_dpp(0, int(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {  // inclusive
+    v = dpp_addu<0x111, 0xf>(v);
+    v = dpp_addu<0x112, 0xf>(v);
+    v = dpp_addu<0x114, 0xf>(v);
+    v = dpp_addu<0x118, 0xf>(v);
+    v = dpp_addu<0x142, 0xa>(v);  // lane 15 of a row into the next row (rows 1 and 3)
+    v = dpp_addu<0x143, 0xc>(v);  // lane 31 into rows 2 and 3
+    return v;
+}
+__device__ __forceinline__ float lane_f32(float v, int src) { return __shfl(v, src, 64); }
+// The value of the lane two away in its group of four, and of the group's lane 0 or 1.
+__device__ __forceinline__ uint32_t other_half(uint32_t v) {
+    return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x4E, 0xf, 0xf, false));
+}
+__device__ __forceinline__ uint32_t first_half(uint32_t v) {
+    return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x44, 0xf, 0xf, false));
+}
+
+// The whole wavefront calls this together; lanes without a walk (live false)
+// only lend themselves to the others' leaf tests.
+// nslab: the slab records of the node arena's children (2 per node),
+// rslab: the root's of this lane's mesh.
+// A step enters at most one internal node and tests at most one leaf per
+// lane, then pops the next entry: the lanes of a wavefront, each at its own
+// place in its own walk, all make progress every step.  About one lane in
+// ten is at a leaf in a step, so the leaf tests of all lanes are dealt out over
+// the wavefront, one triangle a lane, and every owner takes its results in
+// the walk's order: a lane testing its own four triangles ran four tests'
+// instructions every step for a tenth of the lanes.  A step's node records
+// and triangles are loaded together (at clamped addresses, not under their
+// conditions), and the two children's near ties run through one copy of the
+// reference's test.
+// QUAD: four lanes per ray; lanes l and l + 2 of a group keep the same walk
+// and test one child each.  Their state stays equal: both see both results,
+// and only the first half's leaf tests are dealt out.
+template <bool QUAD>
+__device__ __forceinline__ Hit ray_tree(bool live, const MeshRec& m, const NodeRec* __restrict__ nodes,
                                         const RaySlab* __restrict__ nslab, const RaySlab& rslab,
                                         const float* __restrict__ tris, M4 C, f3 o, f3 dir, RayStack& S,
-                                        unsigned long long* err, uint32_t& nbox, uint32_t& ntri, float* sbest,
+                                        unsigned long long* err, uint32_t& nbox, uint32_t& ntri, WalkShared& W,
                                         bool bounded, float eps) {
+    const int lane = S.lane;
+    constexpr int KIDS = QUAD ? 1 : 2;  // children a lane tests itself
+    const uint32_t half = QUAD ? uint32_t(lane >> 1) & 1u : 0u;
     C.m[12] = C.m[12] - o.x;  // centred on the ray origin (Ray.cpp:150-154)
     C.m[13] = C.m[13] - o.y;
     C.m[14] = C.m[14] - o.z;
     C.m[15] = C.m[15] - 0.f;
     Hit best = {false, false, __builtin_huge_valf(), 0.f, 0.f, 0xFFFFFFFFu};
-    publish(sbest, S.lane, __builtin_huge_valf());
+    publish(W.best, lane, __builtin_huge_valf());
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int e = 0; e < 3; ++e) W.ray[3 * k + e][lane] = C.m[4 * k + e];
+    W.ray[12][lane] = dir.x;
+    W.ray[13][lane] = dir.y;
+    W.ray[14][lane] = dir.z;
+    wave_order();
     const LocalRay R = local_ray(C, dir);
-    // the mesh-frame test, or the reference's own where that one is within rounding
-    auto enter = [&](const float* bx, const RaySlab& sl, float& t0, float& t1) -> bool {
-        const int k = box_local(R, bx, sl, t0, t1);
-        if (k != BOX_NEAR) return k == BOX_IN;
+    auto finish = [&]() {  // the walk's end, as the partner lane reads it
+        publish(W.best, lane, (best.hit && best.back) ? best.dist : -1.f);
+    };
+    // the reference's own test of a box whose mesh-frame test is within rounding
+    auto reference = [&](const float* bx, float& t0, float& t1) -> bool {
         return ray_box(dir, xform_box(C, box_from12(bx)), t0, t1) && t1 >= 0.f;
     };
-    float r0, r1;
-    ++nbox;
-    auto finish = [&]() {  // the walk's end, as the partner lane reads it
-        publish(sbest, S.lane, (best.hit && best.back) ? best.dist : -1.f);
-        return best;
-    };
-    if (!enter(m.root.box, rslab, r0, r1)) return finish();
-    if (m.nnodes == 0) {  // the root is a leaf
-        ntri += m.ntri;
-        leaf_hits(tris, m, C, dir, 0, m.ntri, best);
-        return finish();
+    bool active = live;
+    {
+        float r0, r1;
+        const int k = box_local(R, rslab, r0, r1);
+        bool in = k == BOX_IN;
+        if (live && k == BOX_NEAR) in = reference(m.root.box, r0, r1);
+        if (live && half == 0u) ++nbox;
+        active = live && in;
     }
-    const NodeRec* nb = nodes + m.node_base;
+    if (live && !active) finish();
     int sp = 0;
-    // One step enters at most one internal node and tests at most one leaf,
-    // then pops the next entry: the lanes of a wavefront, each at its own
-    // place in its own walk, all make progress every step, where a lane
-    // working through a run of leaves would otherwise hold the others.  Each
-    // lane's sequence of pops, tests and best-hit updates is the walk's own.
-    bool at_node = true;
-    uint32_t node = 0;  // the root, entered without a distance check
-    uint32_t leaf_link = 0, leaf_cnt = 0;
-    for (;;) {
-        if (at_node) {
-            const NodeRec& n = nb[node];
-            float l0, l1, q0, q1;
-            const RaySlab* ns = nslab + 2 * size_t(node);
-            const bool lh = enter(n.c[0].box, ns[0], l0, l1);
-            const bool rh = enter(n.c[1].box, ns[1], q0, q1);
-            nbox += 2;
-            if (sp + 2 > S.cap) {  // deeper than the host allows (it sizes the stack from the tree depths)
-                atomicOr(err, 1ull);
-                best.hit = false;
-                break;
-            }
-            const uint32_t cl = child_cnt(n.c[0]), cr = child_cnt(n.c[1]);
-            // the farther below the nearer (Ray.cpp:175-199); order set by the entry distances alone
-            const bool left_first = !(lh && rh) || l0 < q0;
-            if (lh && rh) {
-                if (left_first) {
-                    S.put(sp++, n.c[1].link, cr, q0);
-                    S.put(sp++, n.c[0].link, cl, l0);
-                } else {
-                    S.put(sp++, n.c[0].link, cl, l0);
-                    S.put(sp++, n.c[1].link, cr, q0);
-                }
-            } else if (lh) {
-                S.put(sp++, n.c[0].link, cl, l0);
-            } else if (rh) {
-                S.put(sp++, n.c[1].link, cr, q0);
-            }
-            at_node = false;
+    const uint32_t node_base = m.node_base, tri_base = m.tri_base;
+    bool at_node = active && m.nnodes != 0;  // the root, entered without a distance check
+    uint32_t node = 0;
+    uint32_t leaf_link = 0, leaf_cnt = active && m.nnodes == 0 ? m.ntri : 0u;  // the root is a leaf
+    while (__ballot(active)) {
+        // the step's node records
+        const size_t ni = at_node ? size_t(node_base) + node : 0;
+        const ChildRec* cr = nodes[ni].c;
+        RaySlab sl[KIDS];
+        uint32_t entry[2];
+#pragma unroll
+        for (int k = 0; k < KIDS; ++k) {
+            sl[k] = nslab[2 * ni + (QUAD ? half : uint32_t(k))];
+            entry[k] = sl[k].entry;
         }
-        if (leaf_cnt) {
-            ntri += leaf_cnt;
-            leaf_hits(tris, m, C, dir, leaf_link, leaf_cnt, best);
-            leaf_cnt = 0;
-            publish(sbest, S.lane, best.dist);
+        // the step's leaf tests, 64 at a time
+        const bool leaves = __ballot(leaf_cnt != 0u) != 0;
+        bool top = false;
+        uint32_t top_entry = 0;
+        float top_t = 0.f;
+        const uint32_t dealt = half == 0u ? leaf_cnt : 0u;
+        uint32_t excl = 0, total = 0;  // this walk's first test
+        uint32_t own = 0, tri = 0;
+        float T[9];
+        auto deal = [&](uint32_t base) {
+            for (uint32_t k = 0; __ballot(k < dealt); ++k) {
+                const uint32_t at = excl + k - base;
+                if (k < dealt && at < 64u) {
+                    W.tri[at] = tri_base + leaf_link + k;
+                    W.own[at] = uint32_t(lane);
+                }
+            }
+            wave_order();
+            const bool in = base + uint32_t(lane) < total;
+            own = in ? W.own[lane] : uint32_t(lane);
+            tri = in ? W.tri[lane] : 0u;
+            wave_order();
+            const float* p = tris + size_t(tri) * 9;
+#pragma unroll
+            for (int e = 0; e < 9; ++e) T[e] = p[e];
+        };
+        if (leaves) {
+            const uint32_t incl = wave_scan_u32(dealt);
+            total = uint32_t(__builtin_amdgcn_readlane(int(incl), 63));
+            excl = QUAD ? first_half(incl - dealt) : incl - dealt;
+            deal(0);
+        }
+        if (__ballot(at_node)) {
+            float t0[2], t1;
+            bool in[2], near[KIDS];
+#pragma unroll
+            for (int k = 0; k < KIDS; ++k) {
+                const int d = box_local(R, sl[k], t0[k], t1);
+                in[k] = d == BOX_IN;
+                near[k] = at_node && d == BOX_NEAR;
+            }
+            if (QUAD) {
+                if (near[0]) in[0] = reference(cr[half].box, t0[0], t1);
+                const bool i = in[0];
+                const float t = t0[0];
+                const uint32_t l = entry[0];
+                const bool oi = other_half(uint32_t(i)) != 0u;
+                const float ot = __uint_as_float(other_half(__float_as_uint(t)));
+                const uint32_t ol = other_half(l);
+                in[0] = half ? oi : i;
+                in[1] = half ? i : oi;
+                t0[0] = half ? ot : t;
+                t0[1] = half ? t : ot;
+                entry[0] = half ? ol : l;
+                entry[1] = half ? l : ol;
+            } else {
+                while (__ballot(near[0] || near[KIDS - 1])) {
+                    if (near[0] || near[KIDS - 1]) {
+                        const bool second = !near[0];
+                        float u0, u1;
+                        const bool hit = reference(cr[second ? 1 : 0].box, u0, u1);
+                        in[0] = second ? in[0] : hit;
+                        in[1] = second ? hit : in[1];
+                        t0[0] = second ? t0[0] : u0;
+                        t0[1] = second ? u0 : t0[1];
+                        near[KIDS - 1] = second ? false : near[KIDS - 1];
+                        near[0] = false;
+                    }
+                }
+            }
+            if (at_node) {
+                nbox += half == 0u ? 2u : 0u;
+                if (sp + 2 > S.cap) {  // deeper than the host allows (it sizes the stack from the tree depths)
+                    atomicOr(err, 1ull);
+                    best.hit = false;
+                    active = false;
+                    sp = 0;
+                } else {
+                    const bool lh = in[0], rh = in[1];
+                    // the farther below the nearer (Ray.cpp:175-199); order set by the entry distances alone
+                    const bool left_first = !(lh && rh) || t0[0] < t0[1];
+                    // the nearer waits in registers: it is the next entry to pop
+                    const bool l = lh && left_first;
+                    if (lh && rh) S.put(sp++, l ? entry[1] : entry[0], l ? t0[1] : t0[0]);
+                    top = lh || rh;
+                    top_entry = l ? entry[0] : entry[1];
+                    top_t = l ? t0[0] : t0[1];
+                }
+                at_node = false;
+            }
+        }
+        if (leaves) {
+            for (uint32_t base = 0;;) {
+                M4 D;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) D.m[4 * k + e] = W.ray[3 * k + e][own];
+                const f3 rd = mk(W.ray[12][own], W.ray[13][own], W.ray[14][own]);
+                float hx = 0.f, hy = 0.f, hd = __builtin_huge_valf();
+                bool hb = false;
+                const bool hit = ray_triangle(rd, mul4(D, mk(T[0], T[1], T[2]), 1.f), mul4(D, mk(T[3], T[4], T[5]), 1.f),
+                                              mul4(D, mk(T[6], T[7], T[8]), 1.f), hx, hy, hd, hb);
+                if (!(hit && hd > 0.f)) hd = __builtin_huge_valf();
+                // every owner takes its triangles in order
+                const uint32_t at0 = excl - base;
+                int win = -1;
+                for (uint32_t k0 = 0; __ballot(k0 < leaf_cnt); k0 += 4) {
+                    float d[4];
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) d[k] = lane_f32(hd, int((at0 + k0 + k) & 63u));
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k)
+                        if (k0 + k < leaf_cnt && at0 + k0 + k < 64u && d[k] < best.dist) {
+                            best.dist = d[k];
+                            best.tri = leaf_link + k0 + k;
+                            win = int(at0 + k0 + k);
+                        }
+                }
+                if (__ballot(win >= 0)) {
+                    const float wx = lane_f32(hx, win & 63), wy = lane_f32(hy, win & 63);
+                    const int wb = __shfl(int(hb), win & 63, 64);
+                    if (win >= 0) {
+                        best.hit = true;
+                        best.back = wb != 0;
+                        best.bx = wx;
+                        best.by = wy;
+                    }
+                }
+                base += 64;
+                if (base >= total) break;
+                deal(base);
+            }
+            if (leaf_cnt) {
+                ntri += dealt;
+                leaf_cnt = 0;
+                publish(W.best, lane, best.dist);
+            }
         }
         // the next entry the best hit so far does not prune
         bool more = false;
-        bool stop = false;
-        const float pb = bounded ? partner(sbest, S.lane) : __builtin_huge_valf();
-        if (pb < 0.f) stop = true;  // the partner ended without a back-face hit
+        const float pb = bounded ? partner(W.best, lane) : __builtin_huge_valf();
+        if (pb < 0.f) {  // the partner ended without a back-face hit
+            sp = 0;
+            top = false;
+        }
         const float bound = (pb + eps) * BOUND_SLACK;
-        while (sp > 0 && !stop) {
-            --sp;
-            const uint32_t ew = S.lc[sp * 64 + S.lane];
-            const uint32_t el = ew & ((1u << RAY_LINK_BITS) - 1u), ec = ew >> RAY_LINK_BITS;
-            const float et = S.t0[sp * 64 + S.lane];
-            if (!(et < best.dist)) continue;
-            if (et > bound) continue;  // no hit in it can make the pass fail
+        // an entry is skipped when the best hit prunes it, or when no hit in it can make the pass fail
+        auto take = [&](uint32_t entry, float et) {
+            if (!(et < best.dist) || et > bound) return;
+            more = true;
+            const uint32_t el = entry & ((1u << RAY_LINK_BITS) - 1u), ec = entry >> RAY_LINK_BITS;
             if (ec == 0u) {
                 node = el;
                 at_node = true;
@@ -400,12 +538,31 @@ __device__ __forceinline__ Hit ray_tree(const MeshRec& m, const NodeRec* __restr
                 leaf_link = el;
                 leaf_cnt = ec;
             }
-            more = true;
-            break;
+        };
+        if (top) take(top_entry, top_t);
+        while (sp > 0 && !more) {  // four entries a look: their LDS reads overlap
+            uint32_t ew[4];
+            float et[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int i = max(sp - 1 - k, 0);
+                ew[k] = S.lc[i * 64 + lane];
+                et[k] = S.t0[i * 64 + lane];
+            }
+            const int n = min(sp, 4);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (k < n && !more) {
+                    --sp;
+                    take(ew[k], et[k]);
+                }
         }
-        if (!more) break;
+        if (!more) {
+            if (live) finish();  // a walk already over publishes the same again
+            active = false;
+        }
     }
-    return finish();
+    return best;
 }
 
 // Ray::MoveOriginEpsilonTowardsDirection (Ray.cpp:13-21).
@@ -450,9 +607,11 @@ __device__ __forceinline__ Hit shfl_hit(const Hit& h, int src) {
     return r;
 }
 
-__device__ __forceinline__ Pass hermann(const MeshView& V, uint32_t meshA, const M4& Amat, uint32_t meshB, const M4& Bmat,
-                        const M3& Bn, f3 o, f3 d, RayStack& S, unsigned long long* err, uint32_t& nbox,
-                        uint32_t& ntri, float* sbest) {
+// The whole wavefront calls it; live: this lane's ray is shot in this pass.
+template <bool QUAD>
+__device__ __forceinline__ Pass hermann(bool live, const MeshView& V, uint32_t meshA, const M4& Amat, uint32_t meshB,
+                                        const M4& Bmat, const M3& Bn, f3 o, f3 d, RayStack& S, unsigned long long* err,
+                                        uint32_t& nbox, uint32_t& ntri, WalkShared& W) {
     Pass r = {false, mk(0.f, 0.f, 0.f), mk(0.f, 0.f, 0.f)};
     const bool own = (threadIdx.x & 1u) != 0;
     const f3 o2 = move_eps(o, d, 4.f);
@@ -461,13 +620,11 @@ __device__ __forceinline__ Pass hermann(const MeshView& V, uint32_t meshA, const
     for (int e = 0; e < 16; ++e) C.m[e] = own ? Amat.m[e] : Bmat.m[e];
     const float eps = vlength(sub(o2, o));
     const uint32_t mesh = own ? meshA : meshB;
-    const MeshRec& mw = V.meshes[mesh];
-    const Hit h = ray_tree(mw, V.nodes, V.slabs + 2 * size_t(mw.node_base), V.roots[mesh], V.tris, C, own ? o2 : o, d, S,
-                           err, nbox, ntri, sbest, own, eps);
+    const Hit h = ray_tree<QUAD>(live, V.meshes[mesh], V.nodes, V.slabs, V.roots[mesh], V.tris, C, own ? o2 : o, d, S, err,
+                           nbox, ntri, W, own, eps);
     const int even = int(threadIdx.x & ~1u);
     const Hit p2 = shfl_hit(h, even), p3 = shfl_hit(h, even + 1);
-    if (!(p2.hit && p2.back)) return r;
-    if (p2.dist <= p3.dist + eps) {
+    if (live && p2.hit && p2.back && p2.dist <= p3.dist + eps) {
         const MeshRec mb = V.meshes[meshB];
         r.ok = true;
         r.response = scale(d, p2.dist);
@@ -505,6 +662,73 @@ __device__ __forceinline__ f3 get3(const float* o) { return mk(o[0], o[1], o[2])
 
 }  // namespace
 
+// Rays of one wavefront: 32 fill its lanes; a call of few rays spreads them
+// over more wavefronts (at least 8 each), as long as these still fit
+// SHOOT_SPREAD, two per SIMD: a wavefront takes as many steps as its longest
+// walk and pays every step for the union of what its lanes need, so fewer
+// walks in each end sooner when the chip has room for them.
+constexpr uint32_t SHOOT_SPREAD = 4096;
+__host__ __device__ inline uint32_t rays_per_wave(uint32_t nrays, uint32_t blocks) {
+    const uint32_t most = blocks < SHOOT_SPREAD ? blocks : SHOOT_SPREAD;
+    return (nrays + 7) / 8 <= most ? 8u : (nrays + 15) / 16 <= most ? 16u : 32u;
+}
+// The rays [r0, r0 + per_wave) of one wavefront, both passes.
+template <bool QUAD>
+__device__ __forceinline__ void shoot_rays(const cd_ray* __restrict__ rays, uint32_t nrays, uint32_t base1,
+                                           const uint32_t* __restrict__ pbegin, uint32_t nq, uint32_t stride,
+                                           const QueryRec* __restrict__ qs, const MeshView& V,
+                                           RayShot* __restrict__ out, uint32_t r0, uint32_t per_wave, RayStack& S,
+                                           unsigned long long* err, uint32_t& nbox, uint32_t& ntri, WalkShared& W) {
+    const uint32_t at = threadIdx.x >> (QUAD ? 2 : 1);  // two or four lanes per ray
+    const uint32_t r = min(r0 + at, nrays - 1);
+    const bool have = at < per_wave && r0 + at < nrays;
+    const int side = r >= base1 ? 1 : 0;
+    const uint32_t local = r - (side ? base1 : 0u);
+    const uint32_t* begin = pbegin + size_t(stride) * side;
+    // the pair: the last one whose rays begin at or before this ray (of equal
+    // begins only the last can hold rays)
+    uint32_t lo = 0, hi = nq;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (begin[mid] <= local) lo = mid;
+        else hi = mid;
+    }
+    const QueryRec q = qs[lo];
+    const M3 Mn = adjoint_transpose(q.rel);
+    RayShot s = {};
+    f3 o = get3(rays[r].origin), d = get3(rays[r].direction);
+    bool live = have;
+    // side 0: first-to-second, then the reflected ray second-to-first; side 1 the other way round
+#pragma unroll 1
+    for (int pass = 0; pass < 2 && __ballot(live); ++pass) {
+        const bool f2s = (pass == 0) == (side == 0);
+        // from the first entity (the identity) at the second (rel), or the other way round
+        M4 A, B;
+        M3 Bn;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const float id = (e % 5 == 0) ? 1.f : 0.f;
+            A.m[e] = f2s ? id : q.rel[e];
+            B.m[e] = f2s ? q.rel[e] : id;
+        }
+#pragma unroll
+        for (int e = 0; e < 9; ++e) Bn.m[e] = f2s ? Mn.m[e] : ((e % 4 == 0) ? 1.f : 0.f);
+        const Pass p = hermann<QUAD>(live, V, f2s ? q.mesh_a : q.mesh_b, A, f2s ? q.mesh_b : q.mesh_a, B, Bn, o, d, S, err,
+                               nbox, ntri, W);
+        live = live && p.ok;
+        if (live) {
+            const f3 F = force_response(p);
+            put3(s.force[pass], f2s ? neg(F) : F);  // sum - F == sum + (-F) exactly
+            put3(s.push[pass], f2s ? neg(p.response) : p.response);
+            s.ok |= 1u << pass;
+            o = add(o, p.response);  // ReflectHermannResult (:104-110)
+            d = neg(p.normal);
+        }
+    }
+    s.pair = lo;
+    if (have && (threadIdx.x & (QUAD ? 3u : 1u)) == 0) out[r] = s;
+}
+
 // Per-ray result: for each of the two passes, the contribution to the summed
 // force response and the push-out vector, as the reference accumulates them
 // (a first-to-second pass subtracts its force and pushes -response, a
@@ -527,58 +751,22 @@ __global__ __launch_bounds__(64) void k_shoot(const cd_ray* __restrict__ rays, u
     // the stacks are sized by the launch: the deepest tree of the call + 2
     // entries per lane, so shallow trees leave LDS for more wavefronts
     extern __shared__ uint32_t s_stack[];
-    __shared__ float s_best[64];  // the lanes' best hits, for the own-tree walks' bound
+    __shared__ WalkShared W;
     uint32_t* base = DEEP ? gstack + size_t(blockIdx.x) * 2 * size_t(stack_entries) * 64 : s_stack;
     RayStack S = {base, reinterpret_cast<float*>(base + stack_entries * 64), int(threadIdx.x), stack_entries};
-    const uint32_t r = (blockIdx.x * blockDim.x + threadIdx.x) >> 1;  // two lanes per ray
     uint32_t nbox = 0, ntri = 0;  // boxes tested, ray-triangle tests: the work counted in ctr->sat, ctr->tritests
     if (dc) {
         base1 = dc[DC_RAYS0];
         nrays = min(nrays, dc[DC_RAYS0] + dc[DC_RAYS1]);
         nq = min(nq, dc[DC_NQ]);
     }
-    if (r < nrays) {  // both lanes of a ray take part or neither
-        const int side = r >= base1 ? 1 : 0;
-        const uint32_t local = r - (side ? base1 : 0u);
-        const uint32_t* begin = pbegin + size_t(stride) * side;
-        // the pair: the last one whose rays begin at or before this ray (of equal
-        // begins only the last can hold rays)
-        uint32_t lo = 0, hi = nq;
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) / 2;
-            if (begin[mid] <= local) lo = mid;
-            else hi = mid;
-        }
-        const QueryRec q = qs[lo];
-        M4 M, I;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            M.m[e] = q.rel[e];
-            I.m[e] = (e % 5 == 0) ? 1.f : 0.f;
-        }
-        const M3 Mn = adjoint_transpose(q.rel);
-        M3 I3;
-#pragma unroll
-        for (int e = 0; e < 9; ++e) I3.m[e] = (e % 4 == 0) ? 1.f : 0.f;
-        RayShot s = {};
-        f3 o = get3(rays[r].origin), d = get3(rays[r].direction);
-        // side 0: first-to-second, then the reflected ray second-to-first; side 1 the other way round
-#pragma unroll 1
-        for (int pass = 0; pass < 2; ++pass) {
-            const bool f2s = (pass == 0) == (side == 0);
-            const Pass p = f2s ? hermann(V, q.mesh_a, I, q.mesh_b, M, Mn, o, d, S, err, nbox, ntri, s_best)
-                               : hermann(V, q.mesh_b, M, q.mesh_a, I, I3, o, d, S, err, nbox, ntri, s_best);
-            if (!p.ok) break;
-            const f3 F = force_response(p);
-            put3(s.force[pass], f2s ? neg(F) : F);  // sum - F == sum + (-F) exactly
-            put3(s.push[pass], f2s ? neg(p.response) : p.response);
-            s.ok |= 1u << pass;
-            o = add(o, p.response);  // ReflectHermannResult (:104-110)
-            d = neg(p.normal);
-        }
-        s.pair = lo;
-        if ((threadIdx.x & 1u) == 0) out[r] = s;
-    }
+    const uint32_t per_wave = rays_per_wave(nrays, gridDim.x);
+    const uint32_t r0 = blockIdx.x * per_wave;
+    if (r0 >= nrays) return;
+    if (per_wave <= 16)
+        shoot_rays<true>(rays, nrays, base1, pbegin, nq, stride, qs, V, out, r0, per_wave, S, err, nbox, ntri, W);
+    else
+        shoot_rays<false>(rays, nrays, base1, pbegin, nq, stride, qs, V, out, r0, per_wave, S, err, nbox, ntri, W);
     // per wavefront, one atomic each
     const unsigned long long bsum = wave_sum_u64(nbox), tsum = wave_sum_u64(ntri);
     if ((threadIdx.x & 63u) == 0) {
@@ -694,14 +882,17 @@ __global__ __launch_bounds__(64) void k_respond(const RayShot* __restrict__ shot
 __global__ void k_ray_slabs(const NodeRec* __restrict__ nodes, uint32_t count, RaySlab* __restrict__ out,
                             const MeshRec* __restrict__ meshes, uint32_t m, RaySlab* __restrict__ root_out) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 2 * count) out[i] = make_slab(nodes[i >> 1].c[i & 1u].box);
-    if (i == 0) *root_out = make_slab(meshes[m].root.box);
+    if (i < 2 * count) out[i] = make_slab(nodes[i >> 1].c[i & 1u]);
+    if (i == 0) *root_out = make_slab(meshes[m].root);
 }
 hipError_t launch_ray_slabs(const NodeRec* nodes, uint32_t count, RaySlab* out, const MeshRec* meshes, uint32_t m,
                             RaySlab* root_out, hipStream_t st) {
     hipLaunchKernelGGL(k_ray_slabs, dim3((2 * count + 255) / 256 + 1), dim3(256), 0, st, nodes, count, out, meshes, m,
                        root_out);
     return hipGetLastError();
+}
+uint32_t shoot_blocks(uint32_t nrays) {
+    return std::max(uint32_t((uint64_t(nrays) + 31) / 32), std::min(uint32_t((uint64_t(nrays) + 7) / 8), SHOOT_SPREAD));
 }
 hipError_t launch_shoot(const cd_ray* rays, uint32_t nrays, uint32_t base1, const uint32_t* pbegin, uint32_t nq,
                         const QueryRec* qs, const MeshRec* meshes, const NodeRec* nodes, const RaySlab* slabs,
@@ -713,8 +904,7 @@ hipError_t launch_shoot(const cd_ray* rays, uint32_t nrays, uint32_t base1, cons
     if (stack_entries < 2) return hipErrorInvalidValue;
     if (!stride) stride = nq;
     const MeshView V = {meshes, nodes, slabs, roots, tris, attrs, vid, nrm, perm};
-    const uint64_t lanes = 2ull * nrays;
-    const dim3 grid(uint32_t((lanes + 63) / 64));
+    const dim3 grid(shoot_blocks(nrays));
     if (stack_entries <= uint32_t(RAY_STACK)) {
         const size_t lds = size_t(stack_entries) * 64 * (sizeof(uint32_t) + sizeof(float));
         hipLaunchKernelGGL(k_shoot<false>, grid, dim3(64), lds, st, rays, nrays, base1, pbegin, nq, stride, dc, qs, V,
