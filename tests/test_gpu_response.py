@@ -221,3 +221,33 @@ def test_step_crowded_scene_grows_its_capacities(mode):
             sc.step()
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("leaf", [1, 4, 13, 64])
+def test_response_of_a_pair_is_its_own(leaf):
+    """A pair's response does not depend on how the call's rays share the
+    wavefronts: over 65,536 rays (32 to a wavefront, two lanes each), over
+    32,768 (16, four lanes each) and of single pairs (8), with leaves whose
+    tests take less or more than a wavefront's 64 lanes, bit for bit."""
+    sc = scenes.Scene(n_entities=256, seed=6, cube=19.0)
+    sc.step()
+    with Collider(leaf_max=leaf) as gpu:
+        ents = sc.entities(gpu.register_soups(sc.soups), ENTITY_DTYPE)
+
+        def shoot(which):
+            gpu.frame(ents[which], MODE_PLAIN)
+            n = len(gpu.uncollide_rays()[1])
+            case(f"response, {len(which)} entities, leaves of {leaf}: {n} rays")
+            return n, {(int(which[r["first"]]), int(which[r["second"]])): r for r in gpu.shoot_rays()}
+
+        n_all, everything = shoot(np.arange(256))
+        n_half, half = shoot(np.arange(170))
+        assert n_all > 65536 >= n_half > 32768
+        singles = {}
+        for i, j in sorted(everything)[:: max(1, len(everything) // 24)]:
+            singles.update(shoot(np.array(sorted((i, j))))[1])
+    for part in (half, singles):
+        assert part
+        for pair, r in part.items():
+            for name in ("shot", "delta", "delta_first", "delta_second"):
+                assert r[name].tobytes() == everything[pair][name].tobytes(), (pair, name)
