@@ -109,8 +109,8 @@ enum { W_QPRE = 0, W_FRONT0, W_FRONT1, W_SMALL, W_SPILL,
        W_ENTS, W_IV, W_K0, W_V0, W_K1, W_V1, W_PAIRS, W_SPAIRS, W_PCOUNT, W_CSORT, W_DUMP0, W_DEFER,
        W_RSTART, W_RPOS, W_RSUMS, W_RCAND, W_RDENSE, W_RCNT, W_RPOS2, W_RHKEY, W_RHVAL, W_RQ, W_RAVG, W_RTOT,
        W_RAYS, W_TASKS, W_SORTT, W_BUD0, W_BUD1, W_BUD2, W_HITS, W_SHOTS, W_RESP, W_PIDS, W_GSTACK,
-       W_SCTR, W_STEPC, W_STEPOUT, W_SEGQ, W_CSEG };
-static_assert(W_CSEG < sizeof(cd_ctx::d_work) / sizeof(DevBuf), "work slots");
+       W_SCTR, W_STEPC, W_STEPOUT, W_SEGQ, W_CSEG, W_NODES };
+static_assert(W_NODES < sizeof(cd_ctx::d_work) / sizeof(DevBuf), "work slots");
 
 RunCounters* dev_counters(cd_ctx* ctx) { return ctx->d_counters.as<RunCounters>(); }
 
@@ -774,6 +774,7 @@ int cd_destroy(cd_ctx* ctx) {
     ctx->h_step.release();
     ctx->h_ents.release();
     ctx->h_ctr.release();
+    ctx->h_nodes.release();
     ctx->d_rayslab.release();
     ctx->d_rootslab.release();
     for (auto& b : ctx->build_scratch) b.release();
@@ -1087,6 +1088,7 @@ int cd_node_global_matrices(cd_ctx* ctx, const cd_node* nodes, uint32_t n, float
     if (n && (!nodes || !global16)) return fail(ctx, CD_E_INVALID, "null node arrays");
     // depth of every node; parents out of range, cycles and chains deeper than 256 are rejected
     constexpr uint32_t MAX_DEPTH = 256;
+    constexpr size_t NODES_KEEP = size_t(64) << 20;  // device bytes kept between calls at most
     std::vector<uint32_t> depth(n, ~0u);
     for (uint32_t i = 0; i < n; ++i) {
         if (!all_finite(nodes[i].local_scale, 13)) return fail(ctx, CD_E_INVALID, "non-finite node transform");
@@ -1094,6 +1096,11 @@ int cd_node_global_matrices(cd_ctx* ctx, const cd_node* nodes, uint32_t n, float
             return fail(ctx, CD_E_INVALID, "node " + std::to_string(i) + ": parent out of range");
     }
     for (uint32_t i = 0; i < n; ++i) {
+        const uint32_t up = nodes[i].parent;
+        if (up == CD_NO_PARENT || depth[up] < MAX_DEPTH) {  // parents first, as hierarchies are stored
+            depth[i] = up == CD_NO_PARENT ? 0u : depth[up] + 1;
+            continue;
+        }
         uint32_t a = i, steps = 0;
         while (depth[a] == ~0u && nodes[a].parent != CD_NO_PARENT) {
             a = nodes[a].parent;
@@ -1113,15 +1120,27 @@ int cd_node_global_matrices(cd_ctx* ctx, const cd_node* nodes, uint32_t n, float
     if (n == 0) return CD_OK;
     (void)hipSetDevice(ctx->device);
     hipStream_t st = ctx->stream;
-    ScopedBuf d_nodes, d_depth, d_out;
-    HCK(ctx, d_nodes.ensure(size_t(n) * sizeof(cd_node)));
-    HCK(ctx, d_depth.ensure(size_t(n) * sizeof(uint32_t)));
-    HCK(ctx, d_out.ensure(size_t(n) * 16 * sizeof(float)));
-    HCK(ctx, hipMemcpyAsync(d_nodes.p, nodes, size_t(n) * sizeof(cd_node), hipMemcpyHostToDevice, st));
-    HCK(ctx, hipMemcpyAsync(d_depth.p, depth.data(), size_t(n) * sizeof(uint32_t), hipMemcpyHostToDevice, st));
-    HCK(ctx, launch_node_globals(d_nodes.as<cd_node>(), d_depth.as<uint32_t>(), n, d_out.as<float>(), st));
-    HCK(ctx, hipMemcpyAsync(global16, d_out.p, size_t(n) * 16 * sizeof(float), hipMemcpyDeviceToHost, st));
+    // the records and their depths in one copy, the matrices in another, both
+    // through pinned memory that the context keeps, as it does the device's
+    // (allocating and freeing three buffers took a third of the call)
+    const size_t rec = size_t(n) * sizeof(cd_node), in = rec + size_t(n) * sizeof(uint32_t);
+    const size_t out_at = (in + 255) & ~size_t(255), res = size_t(n) * 16 * sizeof(float);
+    DevBuf& dev = ctx->d_work[W_NODES];
+    HCK(ctx, dev.ensure(out_at + res));
+    HCK(ctx, ctx->h_nodes.ensure(std::max(in, res)));
+    std::memcpy(ctx->h_nodes.p, nodes, rec);
+    std::memcpy(static_cast<char*>(ctx->h_nodes.p) + rec, depth.data(), size_t(n) * sizeof(uint32_t));
+    float* out = reinterpret_cast<float*>(static_cast<char*>(dev.p) + out_at);
+    HCK(ctx, hipMemcpyAsync(dev.p, ctx->h_nodes.p, in, hipMemcpyHostToDevice, st));
+    HCK(ctx, launch_node_globals(dev.as<cd_node>(), reinterpret_cast<const uint32_t*>(static_cast<char*>(dev.p) + rec),
+                                 n, out, st));
+    HCK(ctx, hipMemcpyAsync(ctx->h_nodes.p, out, res, hipMemcpyDeviceToHost, st));
     HCK(ctx, hipStreamSynchronize(st));
+    std::memcpy(global16, ctx->h_nodes.p, res);
+    if (dev.bytes > NODES_KEEP) {
+        dev.release();
+        ctx->h_nodes.release();
+    }
     return CD_OK;
 }
 
@@ -1502,6 +1521,9 @@ int prepare_rays(cd_ctx* ctx, uint32_t nc, uint32_t stride) {
     return CD_OK;
 }
 
+constexpr uint32_t RAY_TOT_WORDS = 8;  // the totals and, at DC_BIGSEG, the per-query order's flag
+static_assert(DC_BIGSEG < RAY_TOT_WORDS && DC_RAYS1 < RAY_TOT_WORDS, "totals");
+
 // The ray generation on the stream, with no wait: the second side's order of
 // the sorted contacts (unless order_b: already in W_V0), then both sides'
 // candidates, claimed vertices, rays (the second side's after the first's)
@@ -1572,26 +1594,42 @@ int rays_impl(cd_ctx* ctx, cd_pair_rays* pairs, uint32_t pair_cap, uint32_t* n_p
     const uint32_t nc = uint32_t(nc64);
     int rc = prepare_rays(ctx, nc, nq);
     if (rc) return rc;
-    if (!ctx->contacts_sorted) {
-        uint32_t bits[3];
-        contact_field_bits(ctx, nq, bits);
-        HCK(ctx, launch_sort_contacts(ctx->d_contacts.as<cd_contact>(), nc, ctx->d_work[W_CSORT].as<cd_contact>(), bits,
-                                      ctx->d_work[W_K0].as<uint32_t>(), ctx->d_work[W_V0].as<uint32_t>(),
-                                      ctx->d_work[W_K1].as<uint32_t>(), ctx->d_work[W_V1].as<uint32_t>(),
-                                      ctx->d_work[W_SORTT].as<uint32_t>(), st));
-        ctx->contacts_sorted = true;
-    }
     uint32_t* tot = ctx->d_work[W_RTOT].as<uint32_t>();
-    rc = enqueue_rays(ctx, nc, nq, nq, nullptr, nullptr, tot);
-    if (rc) return rc;
-    // one wait, for the totals, the pairs' counts and begins and the averages
-    uint32_t t4[4];
+    uint32_t t4[RAY_TOT_WORDS];
     std::vector<uint32_t> hq(size_t(nq) * 4);
     std::vector<float> ha(size_t(nq) * 6);
-    HCK(ctx, hipMemcpyAsync(t4, tot, sizeof t4, hipMemcpyDeviceToHost, st));
-    HCK(ctx, hipMemcpyAsync(hq.data(), ctx->d_work[W_RQ].p, hq.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    HCK(ctx, hipMemcpyAsync(ha.data(), ctx->d_work[W_RAVG].p, ha.size() * sizeof(float), hipMemcpyDeviceToHost, st));
-    HCK(ctx, hipStreamSynchronize(st));
+    for (;;) {
+        // both orders at once per query, unless a query had more contacts than that ranks
+        uint32_t bits[3];
+        contact_field_bits(ctx, nq, bits);
+        const bool per_query = !ctx->contacts_sorted && !ctx->rays_radix && seg_order_fits(bits[1]);
+        HCK(ctx, launch_fill_u32(tot, RAY_TOT_WORDS, 0u, st));
+        if (per_query) {
+            HCK(ctx, ctx->d_work[W_SEGQ].ensure(size_t(seg_order_words(nq)) * sizeof(uint32_t)));
+            HCK(ctx, ctx->d_work[W_CSEG].ensure(size_t(nc) * sizeof(cd_contact)));
+            uint32_t* qw = ctx->d_work[W_SEGQ].as<uint32_t>();
+            HCK(ctx, launch_fill_u32(qw, nq, 0u, st));
+            HCK(ctx, launch_seg_order(ctx->d_contacts.as<cd_contact>(), nc, nullptr, nq, nullptr, &tot[DC_BIGSEG], qw,
+                                      ctx->d_work[W_CSEG].as<cd_contact>(), ctx->d_work[W_CSORT].as<cd_contact>(),
+                                      ctx->d_work[W_V0].as<uint32_t>(), st));
+        } else if (!ctx->contacts_sorted) {
+            HCK(ctx, launch_sort_contacts(ctx->d_contacts.as<cd_contact>(), nc, ctx->d_work[W_CSORT].as<cd_contact>(),
+                                          bits, ctx->d_work[W_K0].as<uint32_t>(), ctx->d_work[W_V0].as<uint32_t>(),
+                                          ctx->d_work[W_K1].as<uint32_t>(), ctx->d_work[W_V1].as<uint32_t>(),
+                                          ctx->d_work[W_SORTT].as<uint32_t>(), st));
+        }
+        rc = enqueue_rays(ctx, nc, nq, nq, nullptr, nullptr, tot, per_query);
+        if (rc) return rc;
+        // one wait, for the totals, the pairs' counts and begins and the averages
+        HCK(ctx, hipMemcpyAsync(t4, tot, sizeof t4, hipMemcpyDeviceToHost, st));
+        HCK(ctx, hipMemcpyAsync(hq.data(), ctx->d_work[W_RQ].p, hq.size() * sizeof(uint32_t), hipMemcpyDeviceToHost,
+                                st));
+        HCK(ctx, hipMemcpyAsync(ha.data(), ctx->d_work[W_RAVG].p, ha.size() * sizeof(float), hipMemcpyDeviceToHost, st));
+        HCK(ctx, hipStreamSynchronize(st));
+        if (!per_query || !t4[DC_BIGSEG]) break;
+        ctx->rays_radix = true;
+    }
+    ctx->contacts_sorted = true;
     const uint32_t side_rays[2] = {t4[DC_RAYS0], t4[DC_RAYS1]};
     // pairs with rays (CollisionDetection.cpp:63); rays of the first sides, then of the second sides
     std::vector<cd_pair_rays> out;
@@ -1713,7 +1751,7 @@ int ensure_step(cd_ctx* ctx, const StepArgs& a, uint64_t* fcap) {
     HCK(ctx, sort_table(ctx, std::max(std::max(n, P), C), &table));
     HCK(ctx, ctx->d_work[W_SCTR].ensure(sizeof(RunCounters)));
     HCK(ctx, ctx->d_work[W_STEPC].ensure(DC_WORDS * sizeof(uint32_t)));
-    HCK(ctx, ctx->d_work[W_SEGQ].ensure(3 * size_t(P) * sizeof(uint32_t)));
+    HCK(ctx, ctx->d_work[W_SEGQ].ensure(size_t(seg_order_words(P)) * sizeof(uint32_t)));
     HCK(ctx, ctx->d_work[W_CSEG].ensure(size_t(C) * sizeof(cd_contact)));
     if (a.shoot) {
         HCK(ctx, ctx->d_work[W_PIDS].ensure(2 * size_t(P) * sizeof(uint32_t)));
@@ -1776,7 +1814,8 @@ int enqueue_step(cd_ctx* ctx, const StepArgs& a) {
     } else {
         uint32_t* qw3 = ctx->d_work[W_SEGQ].as<uint32_t>();
         HCK(ctx, launch_step_contacts(dev_counters(ctx), ccap, dc, st, qw3, P));
-        HCK(ctx, launch_seg_order(ctx->d_contacts.as<cd_contact>(), C, P, dc, qw3, ctx->d_work[W_CSEG].as<cd_contact>(),
+        HCK(ctx, launch_seg_order(ctx->d_contacts.as<cd_contact>(), C, &dc[DC_NC], P, &dc[DC_NQ], &dc[DC_BIGSEG], qw3,
+                                  ctx->d_work[W_CSEG].as<cd_contact>(),
                                   ctx->d_work[W_CSORT].as<cd_contact>(), v0, st));
     }
     const StepLayout L(P, a.shoot);
@@ -1880,7 +1919,9 @@ int device_run(cd_ctx* ctx, const cd_entity* ents, uint32_t n, bool ref, bool sh
         a.np = ctx->step_np_cap;
         a.nc = ctx->step_nc_cap;
         a.rays = ctx->step_ray_cap;
-        a.radix = ctx->step_radix;
+        uint32_t bits[3];
+        contact_field_bits(ctx, a.np, bits);
+        a.radix = ctx->step_radix || !seg_order_fits(bits[1]);
         a.t = effective_tuning(ctx, a.np);
         uint64_t fcap = 0;
         int rc = ensure_step(ctx, a, &fcap);

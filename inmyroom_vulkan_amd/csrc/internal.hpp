@@ -328,11 +328,13 @@ struct cd_ctx {
     // the tree build's work buffers, kept between builds that need at most
     // BUILD_KEEP bytes of them (a model load builds one document at a time)
     cdk::DevBuf build_scratch[cdk::BUILD_SCRATCH];
+    bool rays_radix = false;  // the same for cd_uncollide_rays after a query batch
     uint32_t step_np_cap = 0, step_nc_cap = 0, step_ray_cap = 0;
     bool step_radix = false;  // a pair had more contacts than the per-pair order ranks: the radix sorts
     hipGraphExec_t step_graph = nullptr, frame_graph = nullptr;  // the whole step; cd_frame's part of it
     std::vector<uint64_t> step_key, frame_key;
     cdk::HostBuf h_step, h_ents;  // the run's result block; its entity records, staged for the graph's upload
     cdk::HostBuf h_ctr;           // a run's counters, read back
+    cdk::HostBuf h_nodes;         // a node hierarchy's records, then its matrices
     hipEvent_t ev[8] = {};
 };

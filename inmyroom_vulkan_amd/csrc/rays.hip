@@ -301,15 +301,16 @@ __global__ void k_ray_count(RaySides b, const QueryRec* __restrict__ qs, const M
                             const uint32_t* __restrict__ perm) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const int side = int(blockIdx.y);
-    if (i >= b.tot[2 * side]) return;
+    const bool valid = i < b.tot[2 * side];
+    if (!__ballot(valid)) return;
     const RayCand* __restrict__ cand = b.dense + size_t(b.n) * side;
     const unsigned long long* __restrict__ hkey = b.hkey + b.H * side;
     const unsigned long long* __restrict__ hval = b.hval + b.H * side;
     const uint64_t hmask = b.H - 1;
     uint32_t* __restrict__ cnt = b.cnt + (size_t(b.n) + 1) * side;
     uint32_t* __restrict__ qcount = b.qw + 2 * size_t(b.qstride) * side;
-    const RayCand r = cand[i];
-    uint32_t k_rays = 1u;  // fallback ray (:155-167)
+    const RayCand r = valid ? cand[i] : RayCand{};
+    uint32_t k_rays = valid ? 1u : 0u;  // fallback ray (:155-167)
     if (r.mask != 0u) {
         const uint32_t mesh = side ? qs[r.query].mesh_b : qs[r.query].mesh_a;
         const MeshRec& m = meshes[mesh];
@@ -319,8 +320,20 @@ __global__ void k_ray_count(RaySides b, const QueryRec* __restrict__ qs, const M
                 claimed(hkey, hval, hmask, vkey(r.query, side, vertex_id(m, attrs[mesh], vid, perm, r.tri, k)), r.tri, k))
                 ++k_rays;
     }
-    cnt[i] = k_rays;
-    atomicAdd(&qcount[r.query], k_rays);
+    if (valid) cnt[i] = k_rays;
+    // The candidates lie query by query: one add per wavefront and query (one
+    // per candidate queued on a few queries' words: 162 us for 64 queries of
+    // some thousand candidates each).
+    const unsigned long long one = __ballot(k_rays & 1u), two = __ballot(k_rays & 2u);
+    unsigned long long todo = __ballot(valid);
+    while (todo) {
+        const int leader = __ffsll(static_cast<long long>(todo)) - 1;
+        const uint32_t q = uint32_t(__shfl(int(r.query), leader, 64));
+        const unsigned long long peers = __ballot(valid && r.query == q);
+        if (int(threadIdx.x & 63u) == leader)
+            atomicAdd(&qcount[q], uint32_t(__popcll(one & peers) + 2 * __popcll(two & peers)));
+        todo &= ~peers;
+    }
 }
 
 __global__ void k_ray_emit(RaySides b, const QueryRec* __restrict__ qs, const MeshRec* __restrict__ meshes,

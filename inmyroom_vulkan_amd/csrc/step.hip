@@ -44,16 +44,23 @@ __global__ __launch_bounds__(1024) void k_step_contacts(const RunCounters* __res
 //  k_seg_count    contacts per pair
 //  k_scan_one     each pair's first slot (and a copy the scatter advances)
 //  k_seg_scatter  every contact into its pair's slots, in any order
-//  k_seg_sort     one workgroup per pair: its contacts' (tri_a, tri_b) keys
-//                 sorted in LDS by a bitonic network (the slot of each in the
-//                 sorted array), then their (tri_b, tri_a) keys with those
-//                 slots (the second order).  A pair of more than SEG_MAX
-//                 contacts sets dc[DC_BIGSEG]; the step then runs again with
-//                 the radix sorts.
+//  k_seg_sort     one workgroup per pair: its contacts ranked by (tri_a,
+//                 tri_b) and by (tri_b, tri_a) together, by merging runs in
+//                 LDS.  Pairs of up to SEG_SMALL contacts take a small workgroup
+//                 each, the larger ones (listed by k_scan_one) a large one; a
+//                 pair of more than SEG_MAX sets a flag, and the caller runs
+//                 the radix sorts instead.
 // The count and the scatter add to a pair's counter once per wavefront and
 // pair (a run's contacts of one pair lie together), not once per contact.
-constexpr uint32_t SEG_MAX = 2048;
-constexpr uint32_t SEG_THREADS = 1024;  // one compare-exchange per thread and stage at SEG_MAX
+// Sorting the two orders one after the other by a bitonic network (66 stages
+// of a barrier and two LDS round trips each for 2,048 contacts) took 38 us in
+// the 512-entity scene, 112 us over 4,099 entities; the query batches and
+// deformables, which used up to 24 radix passes, 0.27-1.2 ms.
+constexpr uint32_t SEG_MAX = 4096, SEG_THREADS = 1024;
+constexpr uint32_t SEG_SMALL = 256;
+constexpr uint32_t SEG_GRID = 1024;   // workgroups of the larger pairs' launch at most
+constexpr uint32_t SEG_TRI_BITS = 25, SEG_POS_BITS = 13;  // a key: both triangles, and the contact's place
+static_assert(2 * SEG_TRI_BITS + SEG_POS_BITS < 64 && SEG_MAX < (1u << SEG_POS_BITS), "key fields");
 
 // Slot of each lane's contact among its pair's (base + rank among the
 // wavefront's lanes of that pair); valid lanes only.  One atomic add per
@@ -61,36 +68,42 @@ constexpr uint32_t SEG_THREADS = 1024;  // one compare-exchange per thread and s
 __device__ __forceinline__ uint32_t seg_slot(uint32_t* __restrict__ ctr, uint32_t q, bool valid) {
     const uint32_t lane = threadIdx.x & 63;
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    unsigned long long todo = __ballot(valid);
-    uint32_t slot = 0;
-    while (todo) {
-        const int leader = __ffsll(static_cast<long long>(todo)) - 1;
-        const uint32_t lq = __shfl(q, leader, 64);
+    unsigned long long todo = __ballot(valid), mine = 0;
+    while (todo) {  // the lanes of each pair the wavefront holds
+        const int first = __ffsll(static_cast<long long>(todo)) - 1;
+        const uint32_t lq = __shfl(q, first, 64);
         const unsigned long long peers = __ballot(valid && q == lq);
-        uint32_t base = 0;
-        if (int(lane) == leader) base = atomicAdd(&ctr[lq], uint32_t(__popcll(peers)));
-        base = __shfl(base, leader, 64);
-        if (valid && q == lq) slot = base + uint32_t(__popcll(peers & below));
+        if (valid && q == lq) mine = peers;
         todo &= ~peers;
     }
+    // the pairs' adds together: one round trip, not one per pair
+    const int leader = valid ? __ffsll(static_cast<long long>(mine)) - 1 : 0;
+    uint32_t base = 0;
+    if (valid && int(lane) == leader) base = atomicAdd(&ctr[q], uint32_t(__popcll(mine)));
+    base = __shfl(base, leader, 64);
+    const uint32_t slot = base + uint32_t(__popcll(mine & below));
     return slot;
 }
 
 __global__ __launch_bounds__(256) void k_seg_count(const cd_contact* __restrict__ c, uint32_t cap,
-                                                   const uint32_t* __restrict__ dc, uint32_t* __restrict__ qcnt) {
+                                                   const uint32_t* __restrict__ nc_dev, uint32_t* __restrict__ qcnt) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = i < min(dc[DC_NC], cap);
+    const bool valid = i < count_of(cap, nc_dev);
     (void)seg_slot(qcnt, valid ? c[i].query : 0u, valid);
 }
 
 // Exclusive scan of n_dev (min with cap) counts in one workgroup, into out
-// and out2.
+// and out2; the counts above SEG_SMALL are listed (large[0] of them, from
+// large[1]), and one above SEG_MAX sets *flag.
 __global__ __launch_bounds__(1024) void k_scan_one(const uint32_t* __restrict__ in, uint32_t cap,
                                                    const uint32_t* __restrict__ n_dev, uint32_t* __restrict__ out,
-                                                   uint32_t* __restrict__ out2) {
+                                                   uint32_t* __restrict__ out2, uint32_t* __restrict__ large,
+                                                   uint32_t* __restrict__ flag) {
     __shared__ uint32_t s_w[16];
+    __shared__ uint32_t s_large;
+    if (threadIdx.x == 0) s_large = 0;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t n = min(*n_dev, cap);
+    const uint32_t n = count_of(cap, n_dev);
     uint32_t carry = 0;
     for (uint32_t base = 0; base < n; base += 1024) {
         const uint32_t i = base + tid;
@@ -111,84 +124,135 @@ __global__ __launch_bounds__(1024) void k_scan_one(const uint32_t* __restrict__ 
         if (i < n) {
             out[i] = carry + before + x - v;
             out2[i] = carry + before + x - v;
+            if (v > SEG_SMALL) large[1 + atomicAdd(&s_large, 1u)] = i;
+            if (v > SEG_MAX) *flag = 1u;
         }
         carry += all;
         __syncthreads();
     }
+    if (tid == 0) large[0] = s_large;
 }
 
 __global__ __launch_bounds__(256) void k_seg_scatter(const cd_contact* __restrict__ c, uint32_t cap,
-                                                     const uint32_t* __restrict__ dc, uint32_t* __restrict__ qfill,
+                                                     const uint32_t* __restrict__ nc_dev, uint32_t* __restrict__ qfill,
                                                      cd_contact* __restrict__ out) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = i < min(dc[DC_NC], cap);
+    const bool valid = i < count_of(cap, nc_dev);
     cd_contact r = {};
     if (valid) r = c[i];
     const uint32_t slot = seg_slot(qfill, r.query, valid);
     if (valid) out[slot] = r;
 }
 
-// Ascending bitonic sort of m (a power of two, up to SEG_MAX) keys with
-// their values in LDS, by the workgroup.
-__device__ __forceinline__ void bitonic_lds(unsigned long long* key, uint32_t* val, uint32_t m) {
-    for (uint32_t k = 2; k <= m; k <<= 1)
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t t = threadIdx.x; t < m / 2; t += blockDim.x) {
-                const uint32_t i = 2 * t - (t & (j - 1)), l = i + j;
-                const unsigned long long ki = key[i], kl = key[l];
-                if ((ki > kl) == ((i & k) == 0)) {
-                    key[i] = kl;
-                    key[l] = ki;
-                    const uint32_t v = val[i];
-                    val[i] = val[l];
-                    val[l] = v;
+// The contacts of one pair, n <= CAP, ranked by both orders.  Runs of L keys
+// are merged into runs of 2 L, every key by a binary search of the run next
+// to it (keys are distinct): each level's searches of all of a thread's keys
+// in both orders are in flight together, and a level costs two barriers.
+template <uint32_t THREADS, uint32_t CAP>
+__device__ __forceinline__ void seg_rank(const cd_contact* __restrict__ seg, uint32_t base, uint32_t n,
+                                         unsigned long long (*key)[CAP], uint32_t* place,
+                                         cd_contact* __restrict__ sorted, uint32_t* __restrict__ order_b) {
+    constexpr uint32_t E = CAP / THREADS;
+    const uint32_t tid = threadIdx.x;
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e) {
+        const uint32_t i = e * THREADS + tid;
+        if (i < n) {
+            const unsigned long long a = seg[base + i].tri_a, b = seg[base + i].tri_b;
+            key[0][i] = (((a << SEG_TRI_BITS) | b) << SEG_POS_BITS) | i;
+            key[1][i] = (((b << SEG_TRI_BITS) | a) << SEG_POS_BITS) | i;
+        }
+    }
+    __syncthreads();
+    for (uint32_t lg = 0, L = 1; L < n; ++lg, L <<= 1) {
+        unsigned long long v[2][E];
+        uint32_t s0[E], len[E], lo[2][E];
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e) {
+            const uint32_t i = min(e * THREADS + tid, n - 1);
+            v[0][e] = key[0][i];
+            v[1][e] = key[1][i];
+            s0[e] = min(((i >> lg) ^ 1u) << lg, n);  // the run next to key i's
+            len[e] = min(L, n - s0[e]);
+            lo[0][e] = lo[1][e] = 0;
+        }
+        for (uint32_t step = L; step > 0; step >>= 1)
+#pragma unroll
+            for (uint32_t e = 0; e < E; ++e) {
+                if (e * THREADS >= n) break;
+                // read whether or not the step stays inside the run: the loads then need no branches
+#pragma unroll
+                for (int o = 0; o < 2; ++o) {
+                    const uint32_t m = lo[o][e] + step;
+                    const unsigned long long k = key[o][min(s0[e] + m, n) - 1];
+                    lo[o][e] = ((m <= len[e]) & (k < v[o][e])) ? m : lo[o][e];
                 }
             }
-            __syncthreads();
+        __syncthreads();
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e) {
+            const uint32_t i = e * THREADS + tid;
+            if (i < n) {
+                const uint32_t at = (((i >> lg) & ~1u) << lg) + (i & (L - 1));
+                key[0][at + lo[0][e]] = v[0][e];
+                key[1][at + lo[1][e]] = v[1][e];
+            }
         }
+        __syncthreads();
+    }
+    // slot r of the sorted array holds contact (key & mask); the second order lists those slots
+    constexpr uint32_t MASK = (1u << SEG_POS_BITS) - 1u;
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e) {
+        const uint32_t r = e * THREADS + tid;
+        if (r < n) {
+            const uint32_t i = uint32_t(key[0][r]) & MASK;
+            place[i] = r;
+            sorted[base + r] = seg[base + i];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e) {
+        const uint32_t r = e * THREADS + tid;
+        if (r < n) order_b[base + r] = base + place[uint32_t(key[1][r]) & MASK];
+    }
+}
+
+__global__ __launch_bounds__(SEG_SMALL) void k_seg_sort_small(const cd_contact* __restrict__ seg,
+                                                       const uint32_t* __restrict__ qoff,
+                                                       const uint32_t* __restrict__ qcnt,
+                                                       const uint32_t* __restrict__ nq_dev, uint32_t cap,
+                                                       cd_contact* __restrict__ sorted, uint32_t* __restrict__ order_b) {
+    __shared__ unsigned long long s_key[2][SEG_SMALL];
+    __shared__ uint32_t s_place[SEG_SMALL];
+    const uint32_t q = blockIdx.x;
+    if (q >= count_of(cap, nq_dev)) return;
+    const uint32_t n = qcnt[q];
+    if (n == 0 || n > SEG_SMALL) return;
+    seg_rank<SEG_SMALL, SEG_SMALL>(seg, qoff[q], n, s_key, s_place, sorted, order_b);
 }
 
 __global__ __launch_bounds__(SEG_THREADS) void k_seg_sort(const cd_contact* __restrict__ seg,
                                                           const uint32_t* __restrict__ qoff,
-                                                          const uint32_t* __restrict__ qcnt, uint32_t* __restrict__ dc,
-                                                          uint32_t cap, cd_contact* __restrict__ sorted,
+                                                          const uint32_t* __restrict__ qcnt,
+                                                          const uint32_t* __restrict__ large,
+                                                          cd_contact* __restrict__ sorted,
                                                           uint32_t* __restrict__ order_b) {
-    __shared__ unsigned long long s_key[SEG_MAX], s_kb[SEG_MAX];  // sort keys; (tri_b, tri_a) of each contact
-    __shared__ uint32_t s_val[SEG_MAX];
-    const uint32_t q = blockIdx.x;
-    if (q >= min(dc[DC_NQ], cap)) return;
-    const uint32_t n = qcnt[q], base = qoff[q];
-    if (n == 0) return;
-    if (n > SEG_MAX) {
-        if (threadIdx.x == 0) dc[DC_BIGSEG] = 1u;
-        return;
-    }
-    uint32_t m = 2;
-    while (m < n) m <<= 1;
-    // keys of the pair's contacts (a run's triangle indices are below 2^25,
-    // so the padding key ~0 sorts after them all)
-    for (uint32_t i = threadIdx.x; i < m; i += blockDim.x) {
-        unsigned long long ka = ~0ull, kb = ~0ull;
-        if (i < n) {
-            const cd_contact& r = seg[base + i];
-            ka = (static_cast<unsigned long long>(r.tri_a) << 32) | r.tri_b;
-            kb = (static_cast<unsigned long long>(r.tri_b) << 32) | r.tri_a;
+    __shared__ unsigned long long s_key[2][SEG_MAX];
+    __shared__ uint32_t s_place[SEG_MAX];
+    for (uint32_t k = blockIdx.x; k < large[0]; k += gridDim.x) {
+        const uint32_t q = large[1 + k], n = qcnt[q];
+        if (n > SEG_MAX) {  // flagged: in any order, so that what follows reads contacts
+            for (uint32_t r = threadIdx.x; r < n; r += SEG_THREADS) {
+                sorted[qoff[q] + r] = seg[qoff[q] + r];
+                order_b[qoff[q] + r] = qoff[q] + r;
+            }
+            continue;
         }
-        s_key[i] = ka;
-        s_kb[i] = kb;
-        s_val[i] = i;
+        seg_rank<SEG_THREADS, SEG_MAX>(seg, qoff[q], n, s_key, s_place, sorted, order_b);
+        __syncthreads();  // the next pair reuses the LDS
     }
-    __syncthreads();
-    bitonic_lds(s_key, s_val, m);
-    // slot r of the sorted array holds contact s_val[r]; the second order
-    // sorts the contacts' (tri_b, tri_a) keys with their slots
-    for (uint32_t r = threadIdx.x; r < n; r += blockDim.x) sorted[base + r] = seg[base + s_val[r]];
-    for (uint32_t r = threadIdx.x; r < m; r += blockDim.x) s_key[r] = r < n ? s_kb[s_val[r]] : ~0ull;
-    __syncthreads();
-    for (uint32_t r = threadIdx.x; r < m; r += blockDim.x) s_val[r] = r;
-    __syncthreads();
-    bitonic_lds(s_key, s_val, m);
-    for (uint32_t r = threadIdx.x; r < n; r += blockDim.x) order_b[base + r] = base + s_val[r];
 }
 
 // One workgroup: each side's counts (qw + 2 stride side) scanned 1024 at a
@@ -243,17 +307,24 @@ hipError_t launch_step_contacts(const RunCounters* ctr, uint64_t cap, uint32_t* 
     hipLaunchKernelGGL(k_step_contacts, dim3(1), dim3(1024), 0, st, ctr, cap, dc, qcnt, np);
     return hipGetLastError();
 }
-hipError_t launch_seg_order(const cd_contact* c, uint32_t nc_cap, uint32_t np_cap, uint32_t* dc, uint32_t* qw3,
-                            cd_contact* seg, cd_contact* sorted, uint32_t* order_b, hipStream_t st) {
-    uint32_t* qcnt = qw3;
-    uint32_t* qoff = qw3 + np_cap;
-    uint32_t* qfill = qw3 + 2 * size_t(np_cap);
+uint32_t seg_order_words(uint32_t np_cap) { return 4 * np_cap + 1; }
+bool seg_order_fits(uint32_t tri_bits) { return tri_bits <= SEG_TRI_BITS; }
+hipError_t launch_seg_order(const cd_contact* c, uint32_t nc_cap, const uint32_t* nc_dev, uint32_t np_cap,
+                            const uint32_t* np_dev, uint32_t* flag, uint32_t* work, cd_contact* seg, cd_contact* sorted,
+                            uint32_t* order_b, hipStream_t st) {
+    uint32_t* qcnt = work;
+    uint32_t* qoff = work + np_cap;
+    uint32_t* qfill = work + 2 * size_t(np_cap);
+    uint32_t* large = work + 3 * size_t(np_cap);
     const dim3 gc((std::max(nc_cap, 1u) + 255) / 256);
-    hipLaunchKernelGGL(k_seg_count, gc, dim3(256), 0, st, c, nc_cap, dc, qcnt);
-    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, st, qcnt, np_cap, dc + DC_NQ, qoff, qfill);
-    hipLaunchKernelGGL(k_seg_scatter, gc, dim3(256), 0, st, c, nc_cap, dc, qfill, seg);
-    hipLaunchKernelGGL(k_seg_sort, dim3(std::max(np_cap, 1u)), dim3(SEG_THREADS), 0, st, seg, qoff, qcnt, dc, np_cap,
+    hipLaunchKernelGGL(k_seg_count, gc, dim3(256), 0, st, c, nc_cap, nc_dev, qcnt);
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, st, qcnt, np_cap, np_dev, qoff, qfill, large, flag);
+    hipLaunchKernelGGL(k_seg_scatter, gc, dim3(256), 0, st, c, nc_cap, nc_dev, qfill, seg);
+    hipLaunchKernelGGL(k_seg_sort_small, dim3(std::max(np_cap, 1u)), dim3(SEG_SMALL), 0, st, seg, qoff, qcnt, np_dev, np_cap,
                        sorted, order_b);
+    // no more pairs than contacts / SEG_SMALL are large
+    const uint32_t gl = std::min(std::min(np_cap, nc_cap / SEG_SMALL), SEG_GRID);
+    if (gl) hipLaunchKernelGGL(k_seg_sort, dim3(gl), dim3(SEG_THREADS), 0, st, seg, qoff, qcnt, large, sorted, order_b);
     return hipGetLastError();
 }
 hipError_t launch_pair_begins(const uint32_t* qw, uint32_t stride, const uint32_t* dc, uint32_t* pbegin, hipStream_t st) {

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from conftest import case
-from inmyroom_vulkan_amd import ENTITY_DTYPE, MODE_BATCHED, MODE_PLAIN, QUERY_DTYPE, scenes
+from inmyroom_vulkan_amd import ENTITY_DTYPE, MODE_BATCHED, MODE_PLAIN, QUERY_DTYPE, Collider, scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -123,3 +123,40 @@ def test_rays_need_a_run(gpu):
             c.uncollide_rays()
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("freq", [1, 3, 6, 12, 20])
+def test_rays_of_a_batch_equal_a_frames(freq):
+    """An icosphere inside a noisy copy of itself, from a few contacts to more
+    than the per-query contact order ranks (4,096; a query above it falls back
+    to the radix sorts a plain frame takes): the same rays, bit for bit."""
+    P, F = scenes.icosphere(freq)
+    rng = np.random.default_rng(7)
+    Q = P * (1.0 + rng.uniform(-0.02, 0.02, (len(P), 1)))
+    with Collider(leaf_max=4) as gpu:
+        a = gpu.register_mesh(P.astype(np.float32), F)
+        b = gpu.register_mesh(Q.astype(np.float32), F)
+        e = np.zeros(2, ENTITY_DTYPE)
+        e["current"] = e["previous"] = [scenes.identity16(), scenes.identity16()]
+        e["mesh_id"] = [a, b]
+        e["should_callback"] = 1
+        gpu.frame(e, MODE_PLAIN)
+        want_pairs, want = gpu.uncollide_rays()
+        a, b = (a, b) if want_pairs[0]["first"] == 0 else (b, a)
+        far = scenes.identity16().copy()
+        far[12] = 9.0  # a query without contacts between two with them
+        for _ in range(2):
+            got_c = gpu.query_batch(gpu.make_queries([a, a, a], [b, b, b], [scenes.identity16(), far,
+                                                                           scenes.identity16()]), MODE_PLAIN)
+            case(f"rays of a query batch, frequency {freq}: {len(got_c)} contacts")
+            assert freq < 20 or len(got_c) > 2 * 4096
+            pairs, rays = gpu.uncollide_rays()
+            assert len(pairs) == 2 * len(want_pairs)
+            n1 = int(pairs["n_first"].sum())
+            for p in pairs:
+                f, s = int(p["begin_first"]), int(p["begin_second"])
+                got = np.concatenate([rays[f : f + p["n_first"]], rays[s : s + p["n_second"]]])
+                assert got.tobytes() == want.tobytes()
+                assert s >= n1
+                for k in ("n_first", "n_second", "avg_first", "avg_second"):
+                    assert p[k].tobytes() == want_pairs[0][k].tobytes(), k
