@@ -31,6 +31,9 @@ constexpr uint32_t TILE_LDS = 64 * (CHUNK_FLOATS + 1);
 // launches cost about 60 us a level, a wavefront about 90 ns a triangle.
 // The level load with 512: 12.7, 1,024: 12.6, 2,048: 13.1 ms.
 constexpr uint32_t BIG_TRIS = 1024;
+// A build takes them when one of its meshes has more than this: below, the
+// one or two levels they would shorten do not pay for their buffers.
+constexpr uint32_t BIG_BUILD = 2048;
 
 struct BigNode {
     uint32_t node, beg, n, tile0;

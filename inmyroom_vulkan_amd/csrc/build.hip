@@ -53,6 +53,7 @@ struct LevelArgs {
     unsigned int* radius_bits;  // one per mesh
     uint32_t leaf_max;
     uint32_t big_min;           // nodes of more triangles than this take the tiled passes
+    uint32_t tiny_max;          // nodes of up to this many (not empty ones) a lane each
 };
 
 constexpr int CHUNK = 256;                 // points per step of the sequential chains
@@ -577,6 +578,10 @@ __device__ __forceinline__ void level_node(const LevelArgs& a, uint32_t ni, uint
 // and runs eig3 on one of them.  Each lane runs the reference's loops as they
 // are written.
 constexpr uint32_t TINY_TRIS = 16;
+// Builds of up to this many triangles keep a wavefront per node throughout:
+// their levels' nodes all run at once, and a second launch a level costs more
+// than it saves (a mesh of 1,280 triangles in a new context 1.5 -> 1.75 ms).
+constexpr uint32_t TINY_BUILD = 16384;
 
 // One triangle's coordinates at a time, TINY_FETCH in flight (indices clamped, as above).
 constexpr uint32_t TINY_FETCH = 3;
@@ -607,7 +612,7 @@ __global__ __launch_bounds__(64) void k_level_tiny(LevelArgs a, uint4* lv) {
             nd = &a.nodes[ni];
             beg = nd->beg;
             n = nd->end - beg;
-            if (n > TINY_TRIS || n == 0) nd = nullptr;  // the other passes' (an empty mesh's root is the wavefronts')
+            if (n > a.tiny_max || n == 0) nd = nullptr;  // the other passes' (an empty mesh's root is the wavefronts')
         }
         if (!nd) n = 0;
         const float* P = a.pos_in + size_t(beg) * 9;
@@ -757,7 +762,7 @@ __global__ __launch_bounds__(64) void k_level(LevelArgs a, uint4* lv) {
     for (uint32_t b = blockIdx.x; b < count; b += gridDim.x) {
         const BNode& nd = a.nodes[first + b];
         const uint32_t n = nd.end - nd.beg;
-        if (n > a.big_min || (n <= TINY_TRIS && n > 0)) continue;
+        if (n > a.big_min || (n <= a.tiny_max && n > 0)) continue;
         level_node(a, first + b, next_first, &lv[1].y, S);
         wave_sync();  // the next node reuses the LDS
     }
@@ -918,9 +923,7 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
     DevBuf* const ids = W + 2;  // ids[0], ids[1]
     DevBuf &pos_fin = W[4], &id_fin = W[5], &nodes = W[6], &mesh_depth = W[7], &level_tab = W[8], &base_nodes = W[9],
            &base_tris = W[10], &slack_bits = W[11], &radius_bits = W[12], &level_list = W[13];
-    DevBuf* const big_list = W + 14;   // big nodes of a level and the next
-    DevBuf* const tile_list = W + 16;  // their tiles
-    DevBuf &big_state = W[18], &tile_sums = W[19], &tile_ext = W[20], &tile_cnt = W[21], &tile_fn = W[22];
+    DevBuf& big_work = W[14];  // all of the tiled passes' arrays: one allocation
     std::vector<BNode> roots(nmesh);
     std::vector<std::pair<uint32_t, uint32_t>> levels;
     std::vector<uint32_t> host_ids;
@@ -930,7 +933,9 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
     uint32_t first = 0, count = nmesh, cur = 0;
     // the roots that take the tiled passes; every level's big nodes are
     // disjoint, so their number and their tiles are bounded once
-    const uint32_t big_min = std::max(BIG_TRIS, ctx->leaf_max);
+    const uint32_t largest = nmesh ? *std::max_element(counts, counts + nmesh) : 0u;
+    const uint32_t big_min = largest > BIG_BUILD ? std::max(BIG_TRIS, ctx->leaf_max) : 0xFFFFFFFFu;
+    const uint32_t tiny_max = T > TINY_BUILD ? TINY_TRIS : 0u;
     std::vector<BigNode> bigs;
     std::vector<uint2> tiles;
     for (uint32_t m = 0; m < nmesh; ++m) {
@@ -939,6 +944,9 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
         bigs.push_back({m, uint32_t(tri_begin[m]), counts[m], uint32_t(tiles.size()) - big_tiles(counts[m])});
     }
     uint32_t nbig = uint32_t(bigs.size()), ntiles = uint32_t(tiles.size());
+    BigArgs big_args{};
+    BigNode* big_list[2] = {};
+    uint2* tile_list[2] = {};
     const size_t big_cap = size_t(T / big_min) + 1, tile_cap = size_t(T / TILE_TRIS) + big_cap;
     const size_t posb = std::max<uint64_t>(T, 1) * 9 * sizeof(float), idb = std::max<uint64_t>(T, 1) * sizeof(uint32_t);
 
@@ -954,17 +962,34 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
     CK(radius_bits.ensure(nmesh * sizeof(uint32_t)));
     CK(level_tab.ensure((LEVEL_BATCH + 1) * sizeof(uint4)));
     if (!bigs.empty()) {
-        CK(big_state.ensure(big_cap * sizeof(BigState)));
-        CK(tile_sums.ensure(tile_cap * sizeof(TileSums)));
-        CK(tile_ext.ensure(tile_cap * sizeof(TileExtents)));
-        CK(tile_cnt.ensure(tile_cap * sizeof(uint4)));
-        CK(tile_fn.ensure(tile_cap * 6 * 128 * sizeof(double2)));
+        size_t at = 0;
+        auto place = [&at](size_t bytes) {
+            const size_t here = at;
+            at += (bytes + 255) & ~size_t(255);
+            return here;
+        };
+        const size_t o_state = place(big_cap * sizeof(BigState)), o_sums = place(tile_cap * sizeof(TileSums)),
+                     o_ext = place(tile_cap * sizeof(TileExtents)), o_cnt = place(tile_cap * sizeof(uint4)),
+                     o_fn = place(tile_cap * 6 * 128 * sizeof(double2));
+        size_t o_big[2], o_tiles[2];
         for (int k = 0; k < 2; ++k) {
-            CK(big_list[k].ensure(big_cap * sizeof(BigNode)));
-            CK(tile_list[k].ensure(tile_cap * sizeof(uint2)));
+            o_big[k] = place(big_cap * sizeof(BigNode));
+            o_tiles[k] = place(tile_cap * sizeof(uint2));
         }
-        CK(hipMemcpyAsync(big_list[0].p, bigs.data(), bigs.size() * sizeof(BigNode), hipMemcpyHostToDevice, st));
-        CK(hipMemcpyAsync(tile_list[0].p, tiles.data(), tiles.size() * sizeof(uint2), hipMemcpyHostToDevice, st));
+        CK(big_work.ensure(at));
+        char* const base = big_work.as<char>();
+        big_args.state = reinterpret_cast<BigState*>(base + o_state);
+        big_args.sums = reinterpret_cast<TileSums*>(base + o_sums);
+        big_args.ext = reinterpret_cast<TileExtents*>(base + o_ext);
+        big_args.counts = reinterpret_cast<uint4*>(base + o_cnt);
+        big_args.fn = reinterpret_cast<double2*>(base + o_fn);
+        big_args.tile_cap = uint32_t(tile_cap);
+        for (int k = 0; k < 2; ++k) {  // a level's big nodes and their tiles, and the next level's
+            big_list[k] = reinterpret_cast<BigNode*>(base + o_big[k]);
+            tile_list[k] = reinterpret_cast<uint2*>(base + o_tiles[k]);
+        }
+        CK(hipMemcpyAsync(big_list[0], bigs.data(), bigs.size() * sizeof(BigNode), hipMemcpyHostToDevice, st));
+        CK(hipMemcpyAsync(tile_list[0], tiles.data(), tiles.size() * sizeof(uint2), hipMemcpyHostToDevice, st));
     }
     CK(base_nodes.ensure(nmesh * sizeof(uint32_t)));
     CK(base_tris.ensure(nmesh * sizeof(uint32_t)));
@@ -999,8 +1024,14 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
         tab[0] = make_uint4(first, count, nbig, ntiles);
         CK(hipMemcpyAsync(level_tab.p, tab.data(), tab.size() * sizeof(uint4), hipMemcpyHostToDevice, st));
         uint64_t big_bound = nbig;
+        // with big nodes about, as many levels as halving the largest there can be takes to end them
+        uint32_t batch = LEVEL_BATCH;
+        if (nbig) {
+            batch = 1;
+            while (batch < LEVEL_BATCH && (uint64_t(ntiles) * TILE_TRIS >> batch) > big_min) ++batch;
+        }
         uint64_t bound = count;
-        for (uint32_t j = 0; j < LEVEL_BATCH; ++j) {
+        for (uint32_t j = 0; j < batch; ++j) {
             LevelArgs a;
             a.nodes = nodes.as<BNode>();
             a.pos_in = pos[cur].as<float>();
@@ -1014,20 +1045,15 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
             a.radius_bits = radius_bits.as<unsigned int>();
             a.leaf_max = ctx->leaf_max;
             a.big_min = big_min;
+            a.tiny_max = tiny_max;
             uint4* const lv = level_tab.as<uint4>() + j;
             if (big_bound) {
-                BigArgs b;
+                BigArgs b = big_args;
                 b.lv = a;
-                b.big = big_list[cur].as<BigNode>();
-                b.tiles = tile_list[cur].as<uint2>();
-                b.big_out = big_list[cur ^ 1].as<BigNode>();
-                b.tiles_out = tile_list[cur ^ 1].as<uint2>();
-                b.state = big_state.as<BigState>();
-                b.sums = tile_sums.as<TileSums>();
-                b.ext = tile_ext.as<TileExtents>();
-                b.counts = tile_cnt.as<uint4>();
-                b.fn = tile_fn.as<double2>();
-                b.tile_cap = uint32_t(tile_cap);
+                b.big = big_list[cur];
+                b.tiles = tile_list[cur];
+                b.big_out = big_list[cur ^ 1];
+                b.tiles_out = tile_list[cur ^ 1];
                 // big nodes at most double per level; a tile list holds at most tile_cap entries
                 const uint32_t gn = uint32_t(std::min<uint64_t>(big_bound, big_cap));
                 const uint32_t gt = uint32_t(std::min<uint64_t>(ntiles + big_bound, tile_cap));
@@ -1044,19 +1070,21 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
             }
             const uint32_t grid = uint32_t(std::min<uint64_t>(bound, LEVEL_GRID));
             hipLaunchKernelGGL(k_level, dim3(grid), dim3(64), 0, st, a, lv);
-            const uint32_t tiny_grid = std::min<uint32_t>(blocks_for(bound, 64), LEVEL_GRID);
-            hipLaunchKernelGGL(k_level_tiny, dim3(tiny_grid), dim3(64), 0, st, a, lv);
-            CK(hipGetLastError());
+            if (tiny_max) {
+                const uint32_t tiny_grid = std::min<uint32_t>(blocks_for(bound, 64), LEVEL_GRID);
+                hipLaunchKernelGGL(k_level_tiny, dim3(tiny_grid), dim3(64), 0, st, a, lv);
+                CK(hipGetLastError());
+            }
             cur ^= 1;
             bound = std::min<uint64_t>(2 * bound, node_cap);
         }
         CK(hipMemcpyAsync(tab.data(), level_tab.p, tab.size() * sizeof(uint4), hipMemcpyDeviceToHost, st));
         CK(hipStreamSynchronize(st));
-        for (uint32_t j = 0; j < LEVEL_BATCH && tab[j].y > 0; ++j) levels.push_back({tab[j].x, tab[j].y});
-        first = tab[LEVEL_BATCH].x;
-        count = tab[LEVEL_BATCH].y;
-        nbig = tab[LEVEL_BATCH].z;
-        ntiles = tab[LEVEL_BATCH].w;
+        for (uint32_t j = 0; j < batch && tab[j].y > 0; ++j) levels.push_back({tab[j].x, tab[j].y});
+        first = tab[batch].x;
+        count = tab[batch].y;
+        nbig = tab[batch].z;
+        ntiles = tab[batch].w;
     }
     {
         const uint32_t total = first;

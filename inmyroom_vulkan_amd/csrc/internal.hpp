@@ -246,7 +246,7 @@ struct RunCounters {
 };
 
 // Build of a batch of triangle soups into the arenas (build.hip).
-constexpr uint32_t BUILD_SCRATCH = 23;
+constexpr uint32_t BUILD_SCRATCH = 15;
 constexpr size_t BUILD_KEEP = size_t(256) << 20;
 
 struct BuildResult {

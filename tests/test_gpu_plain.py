@@ -86,7 +86,7 @@ def _tiled_mesh(kind, n):
 
 @pytest.mark.parametrize("kind", ["grid", "offset", "dyadic", "same", "spread"])
 def test_tree_build_tiled_nodes(gpu, orc, kind):
-    """Nodes above the tiled passes' threshold (1,024 triangles, tiles of 512,
+    """Nodes above the tiled passes' threshold (1,024 triangles in a build with a mesh over 2,048, tiles of 512,
     chunks of 8), around each edge and several in one batch: bit-identical to
     the oracle's sequential sums, and the slack covers the oracle's."""
     sizes = [1024, 1025, 1031, 1536, 1537, 2048, 2049, 3333] + ([] if kind == "same" else [20011])
