@@ -53,7 +53,6 @@ struct LevelArgs {
     unsigned int* radius_bits;  // one per mesh
     uint32_t leaf_max;
     uint32_t big_min;           // nodes of more triangles than this take the tiled passes
-    uint32_t tiny_max;          // nodes of up to this many (not empty ones) a lane each
 };
 
 constexpr int CHUNK = 256;                 // points per step of the sequential chains
@@ -573,15 +572,16 @@ __device__ __forceinline__ void level_node(const LevelArgs& a, uint32_t ni, uint
     if (lane == 0) append_kids(a, nd, nl, next_first, next_count);
 }
 
-// Nodes of few triangles, one lane each: the deepest levels hold most of the
-// nodes, and a wavefront per node of a few triangles leaves most lanes idle
-// and runs eig3 on one of them.  Each lane runs the reference's loops as they
-// are written.
+// Nodes of few triangles, one lane each, on levels of at least TINY_LEVEL
+// nodes: the deepest levels of a large build hold most of its nodes, and a
+// wavefront per node of a few triangles leaves most lanes idle and runs eig3
+// on one of them (level load of 13 meshes: levels of 60,000 nodes 250-450 us,
+// 60-80 a lane each).  A lane takes about 50 us over its node, so smaller
+// levels, whose wavefronts all run at once or nearly so, keep them: 30,000
+// nodes 168 us against 163, 15,000 139 against 136, 2,000 to 8,000 33-57
+// against 80-100.  Each lane runs the reference's loops as they are written.
 constexpr uint32_t TINY_TRIS = 16;
-// Builds of up to this many triangles keep a wavefront per node throughout:
-// their levels' nodes all run at once, and a second launch a level costs more
-// than it saves (a mesh of 1,280 triangles in a new context 1.5 -> 1.75 ms).
-constexpr uint32_t TINY_BUILD = 16384;
+constexpr uint32_t TINY_LEVEL = 32768;
 
 // One triangle's coordinates at a time, TINY_FETCH in flight (indices clamped, as above).
 constexpr uint32_t TINY_FETCH = 3;
@@ -603,6 +603,7 @@ __device__ __forceinline__ void tiny_tris(const float* __restrict__ P, uint32_t 
 
 __global__ __launch_bounds__(64) void k_level_tiny(LevelArgs a, uint4* lv) {
     const uint32_t first = lv[0].x, count = lv[0].y, next_first = first + count;
+    if (count < TINY_LEVEL) return;
     const uint32_t lane = threadIdx.x;
     for (uint32_t b0 = blockIdx.x * 64u; b0 < count; b0 += gridDim.x * 64u) {
         const uint32_t ni = first + b0 + lane;
@@ -612,7 +613,7 @@ __global__ __launch_bounds__(64) void k_level_tiny(LevelArgs a, uint4* lv) {
             nd = &a.nodes[ni];
             beg = nd->beg;
             n = nd->end - beg;
-            if (n > a.tiny_max || n == 0) nd = nullptr;  // the other passes' (an empty mesh's root is the wavefronts')
+            if (n > TINY_TRIS || n == 0) nd = nullptr;  // the other passes' (an empty mesh's root is the wavefronts')
         }
         if (!nd) n = 0;
         const float* P = a.pos_in + size_t(beg) * 9;
@@ -759,10 +760,11 @@ __global__ __launch_bounds__(64) void k_level(LevelArgs a, uint4* lv) {
     const uint32_t first = lv[0].x, count = lv[0].y;
     const uint32_t next_first = first + count;
     if (blockIdx.x == 0 && threadIdx.x == 0) lv[1].x = next_first;
+    const bool tiny = count >= TINY_LEVEL;  // k_level_tiny takes the nodes of few triangles
     for (uint32_t b = blockIdx.x; b < count; b += gridDim.x) {
         const BNode& nd = a.nodes[first + b];
         const uint32_t n = nd.end - nd.beg;
-        if (n > a.big_min || (n <= a.tiny_max && n > 0)) continue;
+        if (n > a.big_min || (tiny && n <= TINY_TRIS && n > 0)) continue;
         level_node(a, first + b, next_first, &lv[1].y, S);
         wave_sync();  // the next node reuses the LDS
     }
@@ -935,7 +937,6 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
     // disjoint, so their number and their tiles are bounded once
     const uint32_t largest = nmesh ? *std::max_element(counts, counts + nmesh) : 0u;
     const uint32_t big_min = largest > BIG_BUILD ? std::max(BIG_TRIS, ctx->leaf_max) : 0xFFFFFFFFu;
-    const uint32_t tiny_max = T > TINY_BUILD ? TINY_TRIS : 0u;
     std::vector<BigNode> bigs;
     std::vector<uint2> tiles;
     for (uint32_t m = 0; m < nmesh; ++m) {
@@ -1045,7 +1046,6 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
             a.radius_bits = radius_bits.as<unsigned int>();
             a.leaf_max = ctx->leaf_max;
             a.big_min = big_min;
-            a.tiny_max = tiny_max;
             uint4* const lv = level_tab.as<uint4>() + j;
             if (big_bound) {
                 BigArgs b = big_args;
@@ -1070,7 +1070,7 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
             }
             const uint32_t grid = uint32_t(std::min<uint64_t>(bound, LEVEL_GRID));
             hipLaunchKernelGGL(k_level, dim3(grid), dim3(64), 0, st, a, lv);
-            if (tiny_max) {
+            if (bound >= TINY_LEVEL) {  // the level's own count decides, on the device
                 const uint32_t tiny_grid = std::min<uint32_t>(blocks_for(bound, 64), LEVEL_GRID);
                 hipLaunchKernelGGL(k_level_tiny, dim3(tiny_grid), dim3(64), 0, st, a, lv);
                 CK(hipGetLastError());

@@ -102,6 +102,27 @@ def test_tree_build_tiled_nodes(gpu, orc, kind):
         assert gpu.mesh_info(mid)["slack"] >= np.float32(tree.slack) * (1 - 1e-6), n
 
 
+def test_tree_build_many_small_meshes(gpu, orc):
+    """33,000 meshes of 0 to 17 triangles: levels wide enough that nodes of up
+    to 16 triangles take a lane each, roots included; one distinct point, flat
+    boxes, ties and index halves among them.  Bit-identical to the oracle."""
+    rng = np.random.default_rng(9)
+    flat = scenes.box_soup()[:2]
+    kinds = [lambda n: rng.normal(size=(n, 9)), lambda n: np.full((n, 9), 0.75),
+             lambda n: np.resize(flat, (n, 9)), lambda n: rng.integers(-2, 3, size=(n, 9)),
+             lambda n: rng.normal(size=(n, 9)) * np.tile([1, 0, 1], 3)]
+    meshes = [kinds[i % 5](i // 5 % 18).astype(np.float32) for i in range(33000)]
+    case(f"tree build, {len(meshes)} meshes of up to 17 triangles")
+    ids = gpu.register_soups(meshes)
+    for k in list(range(180)) + list(range(180, 33000, 411)):
+        tree = orc.tree(meshes[k], 4)
+        want, got = tree.export(), gpu.export_tree(ids[k])
+        for name in ("root", "obbs", "links", "perm"):
+            assert np.asarray(got[name]).tobytes() == np.asarray(want[name]).tobytes(), (k, len(meshes[k]), name)
+        assert gpu.mesh_info(ids[k])["radius"] >= np.sqrt((meshes[k].reshape(-1, 3).astype(np.float64) ** 2)
+                                                          .sum(1).max(initial=0.0)) * (1 - 1e-7)
+
+
 def test_tree_build_hand_derived_splits(gpu_l1, orc):
     """The split cases derived by hand (tie to the left, an axis that leaves a
     side empty, index halves, the larger-surface swap): the GPU build gives
