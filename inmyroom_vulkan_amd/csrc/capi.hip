@@ -109,8 +109,8 @@ enum { W_QPRE = 0, W_FRONT0, W_FRONT1, W_SMALL, W_SPILL,
        W_ENTS, W_IV, W_K0, W_V0, W_K1, W_V1, W_PAIRS, W_SPAIRS, W_PCOUNT, W_CSORT, W_DUMP0, W_DEFER,
        W_RSTART, W_RPOS, W_RSUMS, W_RCAND, W_RDENSE, W_RCNT, W_RPOS2, W_RHKEY, W_RHVAL, W_RQ, W_RAVG, W_RTOT,
        W_RAYS, W_TASKS, W_SORTT, W_BUD0, W_BUD1, W_BUD2, W_HITS, W_SHOTS, W_RESP, W_PIDS, W_GSTACK,
-       W_SCTR, W_STEPC, W_STEPOUT, W_SEGQ, W_CSEG, W_NODES };
-static_assert(W_NODES < sizeof(cd_ctx::d_work) / sizeof(DevBuf), "work slots");
+       W_SCTR, W_STEPC, W_STEPOUT, W_SEGQ, W_CSEG };
+static_assert(W_CSEG < sizeof(cd_ctx::d_work) / sizeof(DevBuf), "work slots");
 
 RunCounters* dev_counters(cd_ctx* ctx) { return ctx->d_counters.as<RunCounters>(); }
 
@@ -775,6 +775,7 @@ int cd_destroy(cd_ctx* ctx) {
     ctx->h_ents.release();
     ctx->h_ctr.release();
     ctx->h_nodes.release();
+    ctx->d_nodemats.release();
     ctx->d_rayslab.release();
     ctx->d_rootslab.release();
     for (auto& b : ctx->build_scratch) b.release();
@@ -1125,7 +1126,7 @@ int cd_node_global_matrices(cd_ctx* ctx, const cd_node* nodes, uint32_t n, float
     // (allocating and freeing three buffers took a third of the call)
     const size_t rec = size_t(n) * sizeof(cd_node), in = rec + size_t(n) * sizeof(uint32_t);
     const size_t out_at = (in + 255) & ~size_t(255), res = size_t(n) * 16 * sizeof(float);
-    DevBuf& dev = ctx->d_work[W_NODES];
+    DevBuf& dev = ctx->d_nodemats;
     HCK(ctx, dev.ensure(out_at + res));
     HCK(ctx, ctx->h_nodes.ensure(std::max(in, res)));
     std::memcpy(ctx->h_nodes.p, nodes, rec);

@@ -335,6 +335,9 @@ struct cd_ctx {
     std::vector<uint64_t> step_key, frame_key;
     cdk::HostBuf h_step, h_ents;  // the run's result block; its entity records, staged for the graph's upload
     cdk::HostBuf h_ctr;           // a run's counters, read back
-    cdk::HostBuf h_nodes;         // a node hierarchy's records, then its matrices
+    // a node hierarchy's records, depths and matrices; not among d_work, whose
+    // addresses key the captured graphs
+    cdk::HostBuf h_nodes;
+    cdk::DevBuf d_nodemats;
     hipEvent_t ev[8] = {};
 };

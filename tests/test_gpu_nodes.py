@@ -5,12 +5,14 @@ GPU, one collision frame over every node with a collision component
 (GameImporter.cpp:320-326), against the oracle's frame on its own decode.
 """
 import os
+import time
 
 import numpy as np
 import pytest
 
 from conftest import GOLDEN, case
-from inmyroom_vulkan_amd import ENTITY_DTYPE, MODE_BATCHED, MODE_PLAIN, NODE_DTYPE, CollideError, GltfDocument
+from inmyroom_vulkan_amd import (ENTITY_DTYPE, MODE_BATCHED, MODE_PLAIN, NODE_DTYPE, Collider, CollideError, GltfDocument,
+                                 scenes)
 from oracle import gltf as og
 from test_nodes import _random_forest
 
@@ -103,3 +105,29 @@ def test_table_room_frame_end_to_end(gpu, orc):
                 g = got[k]
                 assert g["s"].tobytes() == c["s"].tobytes() and g["t"].tobytes() == c["t"].tobytes()
         assert len(want) > 1000
+
+
+def test_node_globals_leave_the_captured_step_alone():
+    """cd_step replays a captured graph; a growing node hierarchy between two
+    steps must not make it capture again (0.2 ms of a step)."""
+    case("steps after node hierarchies of growing size")
+    sc = scenes.Scene(n_entities=64, seed=3, cube=25.0)
+    sc.step()
+    rng = np.random.default_rng(14)
+    with Collider(leaf_max=4) as gpu:
+        ents = sc.entities(gpu.register_soups(sc.soups), ENTITY_DTYPE)
+
+        def step_ms():
+            t = time.perf_counter()
+            gpu.step(ents, MODE_BATCHED)
+            return (time.perf_counter() - t) * 1e3
+
+        for _ in range(3):
+            step_ms()
+        replayed, after = [], []
+        for k in range(8):  # each hierarchy is more than twice the last
+            trs, par = _random_forest(rng, 50 * 3**k, depth_max=4)
+            gpu.node_globals(_records(trs, par))
+            after.append(step_ms())
+            replayed.append(step_ms())
+    assert min(after) < 1.15 * min(replayed), (after, replayed)
