@@ -130,4 +130,40 @@ def test_node_globals_leave_the_captured_step_alone():
             gpu.node_globals(_records(trs, par))
             after.append(step_ms())
             replayed.append(step_ms())
-    assert min(after) < 1.15 * min(replayed), (after, replayed)
+    # a freed address can come back and hide the change of one call, so not the least but the third largest
+    assert sorted(after)[-3] < 1.15 * min(replayed), (after, replayed)
+
+
+def _forest_parents_first(n, seed):
+    rng = np.random.default_rng(seed)
+    q = rng.normal(size=(n, 4))
+    q /= np.linalg.norm(q, axis=1, keepdims=True)
+    trs = np.concatenate([rng.uniform(0.5, 2.0, (n, 3)), q, rng.normal(size=(n, 6))], 1).astype(np.float32)
+    par = (rng.random(n) * np.arange(n)).astype(np.uint32)
+    par[rng.random(n) < 0.02] = 0xFFFFFFFF
+    par[0] = 0xFFFFFFFF
+    return trs, par
+
+
+@pytest.mark.parametrize("n", [1, 30840, 30841, 32768, 32769, 65536, 70001])
+def test_node_globals_around_the_copies_pieces(gpu, orc, n):
+    """Records (68 bytes a node with its depth) and matrices (64) go in pieces of 2 MiB: one, the edges, several."""
+    case(f"node globals, {n} nodes")
+    trs, par = _forest_parents_first(n, n)
+    assert gpu.node_globals(_records(trs, par)).tobytes() == orc.node_globals(trs, par).tobytes()
+
+
+def test_node_globals_time_grows_with_the_nodes():
+    """A large hierarchy's call costs what its nodes do: no more than twice as much a node over 1,000,000 as over 250,000."""
+    case("node globals, 250,000 and 1,000,000 nodes")
+    ms = []
+    with Collider(leaf_max=4) as gpu:
+        for n in (250000, 1000000):
+            nd = _records(*_forest_parents_first(n, 3))
+            t = []
+            for _ in range(5):
+                t0 = time.perf_counter()
+                gpu.node_globals(nd)
+                t.append((time.perf_counter() - t0) * 1e3)
+            ms.append(min(t))
+    assert ms[1] < 8 * ms[0], ms
