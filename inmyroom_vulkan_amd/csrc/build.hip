@@ -1182,8 +1182,10 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
         ctx->tris_used += T;
     }
 fail: {
+        // the tiled passes' arrays, an eighth of the rest at most, are kept or freed with it and don't count:
+        // what a build keeps does not depend on the passes it takes
         size_t kept = 0;
-        for (uint32_t k = 0; k < BUILD_SCRATCH; ++k) kept += W[k].bytes;
+        for (uint32_t k = 0; k < BUILD_SCRATCH; ++k) kept += &W[k] == &big_work ? 0 : W[k].bytes;
         if (!res.err.empty() || kept > BUILD_KEEP)
             for (uint32_t k = 0; k < BUILD_SCRATCH; ++k) W[k].release();
     }

@@ -1,9 +1,10 @@
 """Plain path on the GPU against the oracle, bit for bit (reference semantics)."""
 import numpy as np
 import pytest
+import torch
 
 from conftest import case, golden
-from inmyroom_vulkan_amd import MODE_PLAIN, scenes
+from inmyroom_vulkan_amd import MODE_PLAIN, Collider, scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -100,6 +101,24 @@ def test_tree_build_tiled_nodes(gpu, orc, kind):
         assert np.array_equal(got["links"], want["links"]), n
         assert np.array_equal(got["perm"], want["perm"]), n
         assert gpu.mesh_info(mid)["slack"] >= np.float32(tree.slack) * (1 - 1e-6), n
+
+
+def test_tree_build_keeps_its_buffers():
+    """Work buffers of builds of up to 256 MiB stay with the context, 312 bytes a triangle; the tiled passes' arrays
+    (37 bytes a triangle) do not count, so a mesh of 832,050 triangles (248 MiB without them, 277 with) keeps its."""
+    P, F, _ = scenes.heightfield(646, 200.0, 5.0, seed=2)
+    soup = scenes.soup(P, F)
+    case(f"tree build of {len(soup)} triangles, buffers kept")
+    assert 312 * len(soup) < 256 << 20 < (312 + 36) * len(soup)
+    torch.cuda.synchronize()
+    with Collider(leaf_max=4) as gpu:
+        gpu.register_soups([soup[:1]])
+        free = torch.cuda.mem_get_info()[0]
+        gpu.register_soups([soup])
+        used = free - torch.cuda.mem_get_info()[0]
+        info = gpu.mesh_info(1)
+    arenas = 128 * info["nnodes"] + 44 * len(soup)
+    assert used > arenas + 300 * len(soup), (used, arenas)
 
 
 def test_tree_build_many_small_meshes(gpu, orc):
