@@ -936,7 +936,7 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
     // the roots that take the tiled passes; every level's big nodes are
     // disjoint, so their number and their tiles are bounded once
     const uint32_t largest = nmesh ? *std::max_element(counts, counts + nmesh) : 0u;
-    const uint32_t big_min = largest > BIG_BUILD ? std::max(BIG_TRIS, ctx->leaf_max) : 0xFFFFFFFFu;
+    uint32_t big_min = largest > BIG_BUILD ? std::max(BIG_TRIS, ctx->leaf_max) : 0xFFFFFFFFu;
     std::vector<BigNode> bigs;
     std::vector<uint2> tiles;
     for (uint32_t m = 0; m < nmesh; ++m) {
@@ -977,7 +977,11 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
             o_big[k] = place(big_cap * sizeof(BigNode));
             o_tiles[k] = place(tile_cap * sizeof(uint2));
         }
-        CK(big_work.ensure(at));
+        if (big_work.ensure(at) != hipSuccess) {  // no room for them: a wavefront per node, which needs none
+            (void)hipGetLastError();
+            big_min = 0xFFFFFFFFu;
+            nbig = ntiles = 0;
+        }
         char* const base = big_work.as<char>();
         big_args.state = reinterpret_cast<BigState*>(base + o_state);
         big_args.sums = reinterpret_cast<TileSums*>(base + o_sums);
@@ -989,8 +993,10 @@ BuildResult build_soups(cd_ctx* ctx, const float* tri9, const uint32_t* counts, 
             big_list[k] = reinterpret_cast<BigNode*>(base + o_big[k]);
             tile_list[k] = reinterpret_cast<uint2*>(base + o_tiles[k]);
         }
-        CK(hipMemcpyAsync(big_list[0], bigs.data(), bigs.size() * sizeof(BigNode), hipMemcpyHostToDevice, st));
-        CK(hipMemcpyAsync(tile_list[0], tiles.data(), tiles.size() * sizeof(uint2), hipMemcpyHostToDevice, st));
+        if (nbig) {
+            CK(hipMemcpyAsync(big_list[0], bigs.data(), bigs.size() * sizeof(BigNode), hipMemcpyHostToDevice, st));
+            CK(hipMemcpyAsync(tile_list[0], tiles.data(), tiles.size() * sizeof(uint2), hipMemcpyHostToDevice, st));
+        }
     }
     CK(base_nodes.ensure(nmesh * sizeof(uint32_t)));
     CK(base_tris.ensure(nmesh * sizeof(uint32_t)));
