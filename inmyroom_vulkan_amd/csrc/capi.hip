@@ -1779,10 +1779,8 @@ int ensure_step(cd_ctx* ctx, const StepArgs& a, uint64_t* fcap) {
         HCK(ctx, ctx->d_work[W_PIDS].ensure(2 * size_t(P) * sizeof(uint32_t)));
         HCK(ctx, ctx->d_work[W_SHOTS].ensure(size_t(R) * sizeof(RayShot)));
         HCK(ctx, ctx->d_work[W_RESP].ensure(size_t(P) * sizeof(cd_pair_response)));
-        if (a.stack_entries > uint32_t(RAY_STACK_ENTRIES)) {  // trees deeper than the LDS stack holds
-            const size_t blocks = shoot_blocks(uint32_t(R));
-            HCK(ctx, ctx->d_work[W_GSTACK].ensure(blocks * 2 * a.stack_entries * 64 * sizeof(uint32_t)));
-        }
+        if (shoot_deep(a.stack_entries))  // trees deeper than the LDS stack holds
+            HCK(ctx, ctx->d_work[W_GSTACK].ensure(shoot_gstack_bytes(R, a.stack_entries)));
     }
     const StepLayout L(P, a.shoot);
     HCK(ctx, ctx->d_work[W_STEPOUT].ensure(size_t(L.words) * sizeof(uint32_t)));
@@ -1865,7 +1863,7 @@ int enqueue_step(cd_ctx* ctx, const StepArgs& a) {
     uint32_t* qw = ctx->d_work[W_RQ].as<uint32_t>();
     uint32_t* pbegin = ctx->d_work[W_PIDS].as<uint32_t>();
     RunCounters* sctr = ctx->d_work[W_SCTR].as<RunCounters>();
-    uint32_t* gstack = a.stack_entries > uint32_t(RAY_STACK_ENTRIES) ? ctx->d_work[W_GSTACK].as<uint32_t>() : nullptr;
+    uint32_t* gstack = shoot_deep(a.stack_entries) ? ctx->d_work[W_GSTACK].as<uint32_t>() : nullptr;
     HCK(ctx, launch_pair_begins(qw, P, dc, pbegin, st));
     HCK(ctx, launch_zero(sctr, st));
     HCK(ctx, launch_shoot(ctx->d_work[W_RAYS].as<cd_ray>(), R, 0, pbegin, P, dq, dm, ctx->d_nodes.as<NodeRec>(),
@@ -2160,9 +2158,8 @@ int cd_shoot_rays(cd_ctx* ctx, const cd_shoot_params* params, cd_pair_response* 
     const uint32_t* qw = ctx->d_work[W_RQ].as<uint32_t>();
     const uint32_t* pbegin = ctx->d_work[W_PIDS].as<uint32_t>() + 2 * size_t(nq);
     uint32_t* gstack = nullptr;  // trees deeper than the LDS stack holds: the stacks in HBM
-    if (stack_entries > uint32_t(RAY_STACK_ENTRIES)) {
-        const size_t blocks = shoot_blocks(uint32_t(ctx->ray_total));
-        HCK(ctx, ctx->d_work[W_GSTACK].ensure(blocks * 2 * stack_entries * 64 * sizeof(uint32_t)));
+    if (shoot_deep(stack_entries)) {
+        HCK(ctx, ctx->d_work[W_GSTACK].ensure(shoot_gstack_bytes(uint32_t(ctx->ray_total), stack_entries)));
         gstack = ctx->d_work[W_GSTACK].as<uint32_t>();
     }
     {

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "internal.hpp"
+#include "shootshape.hpp"
 #include "sortbits.hpp"
 
 namespace cdk {
@@ -108,15 +109,17 @@ hipError_t launch_sort_perm(const cd_contact* in, uint32_t n, int f_hi, int f_mi
 // response.hip
 // pbegin: per side (nq each) the first ray of every pair, non-decreasing;
 // stack_entries: the deepest tree the rays meet + 2; above RAY_STACK_ENTRIES
-// the stacks live in gstack, shoot_blocks(nrays) * 2 * stack_entries * 64
-// words; ctr->err gets bit 0 if a traversal stack would have overflowed,
+// the stacks live in gstack, shoot_gstack_bytes(nrays, stack_entries) bytes; ctr->err gets bit 0 if a traversal stack would have overflowed,
 // ctr->sat the boxes tested and ctr->tritests the ray-triangle tests.
 // stride: the per-side spacing of pbegin (0: nq); dc: the step's count block
 // (DC_*), from which the ray and pair counts are read when given, nrays and
 // nq being the capacities.
 // slabs / roots: the slab records of every node's children and every mesh's
 // root (launch_ray_slabs), current for the meshes the rays meet.
-uint32_t shoot_blocks(uint32_t nrays);  // wavefronts of a launch over nrays rays
+constexpr bool shoot_deep(uint32_t stack_entries) { return stack_entries > uint32_t(RAY_STACK_ENTRIES); }
+constexpr size_t shoot_gstack_bytes(uint32_t nrays, uint32_t stack_entries) {
+    return shoot_blocks(nrays, stack_entries, true) * shoot_stack_bytes(stack_entries);
+}
 hipError_t launch_shoot(const cd_ray* rays, uint32_t nrays, uint32_t base1, const uint32_t* pbegin, uint32_t nq,
                         const QueryRec* qs, const MeshRec* meshes, const NodeRec* nodes, const RaySlab* slabs,
                         const RaySlab* roots, const float* tris,

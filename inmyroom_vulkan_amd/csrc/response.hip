@@ -21,7 +21,6 @@
 // distance is not negative and, when it is popped, its entry distance is
 // below the best hit so far: the nodes visited, and the order in which equal
 // distances are met, are those of the reference's recursion.
-#include <algorithm>
 
 #include "rayattr.hpp"
 
@@ -30,7 +29,6 @@ namespace cdk {
 namespace {
 
 constexpr float FLT_EPS = 1.1920928955078125e-07f;  // std::numeric_limits<float>::epsilon()
-constexpr int RAY_STACK = RAY_STACK_ENTRIES;  // entries per lane: a tree's depth + 2
 
 __device__ __forceinline__ float max_std(float a, float b) { return (a < b) ? b : a; }  // std::max
 __device__ __forceinline__ float min_std(float a, float b) { return (b < a) ? b : a; }  // std::min
@@ -662,16 +660,6 @@ __device__ __forceinline__ f3 get3(const float* o) { return mk(o[0], o[1], o[2])
 
 }  // namespace
 
-// Rays of one wavefront: 32 fill its lanes; a call of few rays spreads them
-// over more wavefronts (at least 8 each), as long as these still fit
-// SHOOT_SPREAD, two per SIMD: a wavefront takes as many steps as its longest
-// walk and pays every step for the union of what its lanes need, so fewer
-// walks in each end sooner when the chip has room for them.
-constexpr uint32_t SHOOT_SPREAD = 4096;
-__host__ __device__ inline uint32_t rays_per_wave(uint32_t nrays, uint32_t blocks) {
-    const uint32_t most = blocks < SHOOT_SPREAD ? blocks : SHOOT_SPREAD;
-    return (nrays + 7) / 8 <= most ? 8u : (nrays + 15) / 16 <= most ? 16u : 32u;
-}
 // The rays [r0, r0 + per_wave) of one wavefront, both passes.
 template <bool QUAD>
 __device__ __forceinline__ void shoot_rays(const cd_ray* __restrict__ rays, uint32_t nrays, uint32_t base1,
@@ -891,9 +879,6 @@ hipError_t launch_ray_slabs(const NodeRec* nodes, uint32_t count, RaySlab* out, 
                        root_out);
     return hipGetLastError();
 }
-uint32_t shoot_blocks(uint32_t nrays) {
-    return std::max(uint32_t((uint64_t(nrays) + 31) / 32), std::min(uint32_t((uint64_t(nrays) + 7) / 8), SHOOT_SPREAD));
-}
 hipError_t launch_shoot(const cd_ray* rays, uint32_t nrays, uint32_t base1, const uint32_t* pbegin, uint32_t nq,
                         const QueryRec* qs, const MeshRec* meshes, const NodeRec* nodes, const RaySlab* slabs,
                         const RaySlab* roots, const float* tris,
@@ -904,8 +889,9 @@ hipError_t launch_shoot(const cd_ray* rays, uint32_t nrays, uint32_t base1, cons
     if (stack_entries < 2) return hipErrorInvalidValue;
     if (!stride) stride = nq;
     const MeshView V = {meshes, nodes, slabs, roots, tris, attrs, vid, nrm, perm};
-    const dim3 grid(shoot_blocks(nrays));
-    if (stack_entries <= uint32_t(RAY_STACK)) {
+    const bool deep = shoot_deep(stack_entries);
+    const dim3 grid(shoot_blocks(nrays, stack_entries, deep));
+    if (!deep) {
         const size_t lds = size_t(stack_entries) * 64 * (sizeof(uint32_t) + sizeof(float));
         hipLaunchKernelGGL(k_shoot<false>, grid, dim3(64), lds, st, rays, nrays, base1, pbegin, nq, stride, dc, qs, V,
                            shots, int(stack_entries), ctr, (uint32_t*)nullptr);
