@@ -1144,7 +1144,7 @@ int cd_node_global_matrices(cd_ctx* ctx, const cd_node* nodes, uint32_t n, float
         if (len > from_rec)
             std::memcpy(h + from_rec, reinterpret_cast<const char*>(depth.data()) + (at + from_rec - rec), len - from_rec);
         HCK(ctx, hipMemcpyAsync(d + at, h, len, hipMemcpyHostToDevice, st));
-        HCK(ctx, hipEventRecord(arrived[k & 1], st));
+        if (at + 2 * half < in) HCK(ctx, hipEventRecord(arrived[k & 1], st));
     }
     HCK(ctx, launch_node_globals(dev.as<cd_node>(), reinterpret_cast<const uint32_t*>(d + rec), n,
                                  reinterpret_cast<float*>(d + out_at), st));
@@ -1153,12 +1153,12 @@ int cd_node_global_matrices(cd_ctx* ctx, const cd_node* nodes, uint32_t n, float
         if (at >= res) return hipSuccess;
         hipError_t e = hipMemcpyAsync(stage + (k & 1) * half, d + out_at + at, std::min(half, res - at),
                                       hipMemcpyDeviceToHost, st);
-        return e == hipSuccess ? hipEventRecord(arrived[k & 1], st) : e;
+        return e == hipSuccess && at + half < res ? hipEventRecord(arrived[k & 1], st) : e;
     };
     HCK(ctx, fetch(0));  // after the uploads that read this half, in stream order
     HCK(ctx, fetch(1));
     for (size_t k = 0; k * half < res; ++k) {
-        HCK(ctx, hipEventSynchronize(arrived[k & 1]));
+        HCK(ctx, (k + 1) * half < res ? hipEventSynchronize(arrived[k & 1]) : hipStreamSynchronize(st));
         std::memcpy(reinterpret_cast<char*>(global16) + k * half, stage + (k & 1) * half, std::min(half, res - k * half));
         HCK(ctx, fetch(k + 2));
     }

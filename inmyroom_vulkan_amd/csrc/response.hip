@@ -21,7 +21,6 @@
 // distance is not negative and, when it is popped, its entry distance is
 // below the best hit so far: the nodes visited, and the order in which equal
 // distances are met, are those of the reference's recursion.
-
 #include "rayattr.hpp"
 
 namespace cdk {
