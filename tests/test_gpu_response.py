@@ -168,35 +168,64 @@ def test_step_equals_frame_rays_and_shoot(mode, step_graph):
         gpu.close()
 
 
-@pytest.mark.parametrize("step_graph", [0, 2])
-def test_step_pair_beyond_per_pair_order(step_graph):
-    """An icosphere inside a copy of itself with seeded radial noise: the two
-    surfaces cross all over, one pair with more contacts than the step's
-    per-pair contact order ranks (2,048).  The step runs again with the radix
-    sorts and still gives the three calls' records, bit for bit."""
-    case(f"cd_step, one pair beyond the per-pair contact order, step_graph {step_graph}")
-    P, F = scenes.icosphere(12)
+def _noisy_spheres(gpu, freq):
+    """Two entities: an icosphere inside a copy of itself with seeded radial
+    noise; the two surfaces cross all over."""
+    P, F = scenes.icosphere(freq)
     rng = np.random.default_rng(7)
     Q = P * (1.0 + rng.uniform(-0.02, 0.02, (len(P), 1)))
-    gpu = Collider(leaf_max=4)
-    try:
+    e = np.zeros(2, ENTITY_DTYPE)
+    e["current"] = [scenes.identity16(), scenes.identity16()]
+    e["previous"] = [_tmat(-0.2), scenes.identity16()]
+    e["mesh_id"] = [gpu.register_mesh(P.astype(np.float32), F), gpu.register_mesh(Q.astype(np.float32), F)]
+    e["should_callback"] = 1
+    return e
+
+
+@pytest.mark.parametrize("mode", [MODE_REFERENCE, MODE_BATCHED])
+@pytest.mark.parametrize("step_graph", [0, 2])
+def test_step_pair_beyond_per_pair_order(step_graph, mode):
+    """One pair with more contacts than the step's per-pair contact order
+    ranks (4,096).  The step is the context's first call, so what its first
+    attempt leaves in the order's buffers is all there is in them; it runs
+    again with the radix sorts and gives the three calls' records, bit for
+    bit, and so does the next step."""
+    case(f"cd_step, one pair beyond the per-pair contact order, step_graph {step_graph}, mode {mode}")
+    with Collider(leaf_max=4) as gpu:
         gpu.set_tuning(step_graph=step_graph)
-        a = gpu.register_mesh(P.astype(np.float32), F)
-        b = gpu.register_mesh(Q.astype(np.float32), F)
+        e = _noisy_spheres(gpu, 16)
+        got = [gpu.step(e, mode) for _ in range(2)]
+        pairs, _ = gpu.frame(e, mode)
+        assert len(pairs) == 1 and int(pairs[0]["contact_count"]) > 6000, pairs
+        gpu.uncollide_rays()
+        want = gpu.shoot_rays()
+        assert len(want) == 1
+        for g in got:
+            assert g.tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("contacts", [255, 256, 257, 4095, 4096, 4097])
+def test_step_contact_order_limits(contacts):
+    """A pair whose contacts just fit the order's small workgroups (256), its
+    large ones (4,096), or neither: the step's records are the three calls'.
+    A comb of thin triangles through a plate of one: a contact a tooth."""
+    case(f"cd_step, one pair of {contacts} contacts")
+    x = np.arange(contacts, dtype=np.float64) * 0.01 + 0.5
+    comb = np.zeros((contacts, 9))
+    comb[:, 0], comb[:, 2], comb[:, 3], comb[:, 5], comb[:, 6], comb[:, 8] = x, -1.0, x + 0.004, -1.0, x + 0.002, 1.0
+    comb[:, 1] = comb[:, 4] = comb[:, 7] = 0.25
+    plate = np.array([[-100.0, -100.0, 0.0, 200.0, -100.0, 0.0, 0.0, 300.0, 0.0]])
+    with Collider(leaf_max=4) as gpu:
         e = np.zeros(2, ENTITY_DTYPE)
         e["current"] = [scenes.identity16(), scenes.identity16()]
         e["previous"] = [_tmat(-0.2), scenes.identity16()]
-        e["mesh_id"] = [a, b]
+        e["mesh_id"] = gpu.register_soups([comb.astype(np.float32), plate.astype(np.float32)])
         e["should_callback"] = 1
-        for mode in (MODE_REFERENCE, MODE_BATCHED):
-            pairs, _ = gpu.frame(e, mode)
-            assert len(pairs) == 1 and int(pairs[0]["contact_count"]) > 2048, pairs
-            gpu.uncollide_rays()
-            want = gpu.shoot_rays()
-            got = gpu.step(e, mode)
-            assert len(got) == 1 and got.tobytes() == want.tobytes(), mode
-    finally:
-        gpu.close()
+        got = gpu.step(e, MODE_BATCHED)
+        pairs, _ = gpu.frame(e, MODE_BATCHED)
+        assert int(pairs[0]["contact_count"]) == contacts
+        gpu.uncollide_rays()
+        assert got.tobytes() == gpu.shoot_rays().tobytes()
 
 
 @pytest.mark.parametrize("mode", [MODE_REFERENCE, MODE_BATCHED])
