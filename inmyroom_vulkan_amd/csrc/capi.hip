@@ -1543,8 +1543,8 @@ int prepare_rays(cd_ctx* ctx, uint32_t nc, uint32_t stride) {
     return CD_OK;
 }
 
-constexpr uint32_t RAY_TOT_WORDS = 8;  // the totals and, at DC_BIGSEG, the per-query order's flag
-static_assert(DC_BIGSEG < RAY_TOT_WORDS && DC_RAYS1 < RAY_TOT_WORDS, "totals");
+constexpr uint32_t RAY_TOT_WORDS = 16;  // the totals and the flags, at the step's places (DC_BIGSEG, DC_PROBE)
+static_assert(DC_PROBE < RAY_TOT_WORDS && DC_BIGSEG < RAY_TOT_WORDS && DC_RAYS1 < RAY_TOT_WORDS, "totals");
 
 // The ray generation on the stream, with no wait: the second side's order of
 // the sorted contacts (unless order_b: already in W_V0), then both sides'
@@ -1651,6 +1651,7 @@ int rays_impl(cd_ctx* ctx, cd_pair_rays* pairs, uint32_t pair_cap, uint32_t* n_p
         if (!per_query || !t4[DC_BIGSEG]) break;
         ctx->rays_radix = true;
     }
+    if (t4[DC_PROBE]) return fail(ctx, CD_E_HIP, "ray generation: vertex set full");
     ctx->contacts_sorted = true;
     const uint32_t side_rays[2] = {t4[DC_RAYS0], t4[DC_RAYS1]};
     // pairs with rays (CollisionDetection.cpp:63); rays of the first sides, then of the second sides
@@ -1992,6 +1993,7 @@ int device_run(cd_ctx* ctx, const cd_entity* ents, uint32_t n, bool ref, bool sh
         }
         if (retry) continue;
         if (sh.err) return fail(ctx, CD_E_STACK, "ray traversal stack overflow");
+        if (dcw[DC_PROBE]) return fail(ctx, CD_E_HIP, "ray generation: vertex set full");
         // what the separate calls would leave: the pairs, sorted contacts (and rays) of the frame
         const uint32_t nq = dcw[DC_NQ];
         const uint2* hp = reinterpret_cast<const uint2*>(w + L->pairs);

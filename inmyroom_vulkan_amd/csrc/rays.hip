@@ -258,7 +258,9 @@ __global__ void k_compact(RaySides b) {
 
 // Hash set of claimed vertices: key (query, side, vertex id), value the
 // smallest (triangle << 2 | corner) that wants the vertex.  Linear probing in
-// a power-of-two table with more slots than keys, so every probe ends.
+// a power-of-two table with more slots than keys, so every probe ends at its
+// key or a free slot; one that has seen every slot all the same sets
+// tot[DC_PROBE], and the call fails instead of never ending.
 __device__ __forceinline__ uint64_t vkey(uint32_t query, int side, uint32_t v) {
     return (uint64_t(query) << 33) | (uint64_t(side) << 32) | uint64_t(v);
 }
@@ -279,20 +281,30 @@ __global__ void k_vert_claim(RaySides b, const QueryRec* __restrict__ qs, const 
     for (int k = 0; k < 3; ++k) {
         if (!(r.mask & (1u << k))) continue;
         const uint64_t key = vkey(r.query, side, vertex_id(m, attrs[mesh], vid, perm, r.tri, k));
-        uint64_t h = mix64(key) & hmask;
+        uint64_t h = mix64(key) & hmask, left = hmask;
         for (;;) {
             const unsigned long long prev = atomicCAS(&hkey[h], static_cast<unsigned long long>(EMPTY),
                                                       static_cast<unsigned long long>(key));
             if (prev == EMPTY || prev == key) break;
+            if (left-- == 0) {
+                b.tot[DC_PROBE] = 1u;
+                return;
+            }
             h = (h + 1) & hmask;
         }
         atomicMin(&hval[h], (static_cast<unsigned long long>(r.tri) << 2) | static_cast<unsigned long long>(k));
     }
 }
 __device__ __forceinline__ bool claimed(const unsigned long long* hkey, const unsigned long long* hval, uint64_t hmask,
-                                        uint64_t key, uint32_t tri, int k) {
-    uint64_t h = mix64(key) & hmask;
-    while (hkey[h] != key) h = (h + 1) & hmask;  // present: inserted by k_vert_claim
+                                        uint64_t key, uint32_t tri, int k, uint32_t* tot) {
+    uint64_t h = mix64(key) & hmask, left = hmask;
+    while (hkey[h] != key) {  // present: inserted by k_vert_claim
+        if (left-- == 0) {
+            tot[DC_PROBE] = 1u;
+            return false;
+        }
+        h = (h + 1) & hmask;
+    }
     return hval[h] == ((static_cast<unsigned long long>(tri) << 2) | static_cast<unsigned long long>(k));
 }
 
@@ -317,7 +329,8 @@ __global__ void k_ray_count(RaySides b, const QueryRec* __restrict__ qs, const M
         k_rays = 0u;
         for (int k = 0; k < 3; ++k)
             if ((r.mask & (1u << k)) &&
-                claimed(hkey, hval, hmask, vkey(r.query, side, vertex_id(m, attrs[mesh], vid, perm, r.tri, k)), r.tri, k))
+                claimed(hkey, hval, hmask, vkey(r.query, side, vertex_id(m, attrs[mesh], vid, perm, r.tri, k)), r.tri, k,
+                        b.tot))
                 ++k_rays;
     }
     if (valid) cnt[i] = k_rays;
@@ -372,7 +385,7 @@ __global__ void k_ray_emit(RaySides b, const QueryRec* __restrict__ qs, const Me
         for (int k = 0; k < 3; ++k) {
             if (!(r.mask & (1u << k))) continue;
             const uint32_t v = vertex_id(m, attr, vid, perm, r.tri, k);
-            if (!claimed(hkey, hval, hmask, vkey(r.query, side, v), r.tri, k)) continue;
+            if (!claimed(hkey, hval, hmask, vkey(r.query, side, v), r.tri, k, b.tot)) continue;
             const f3 n = corner_normal(attr, nrm, v, t9);
             const f3 nn = side ? normalize(mul3(NM, n)) : normalize(n);  // Triangle.cpp:180-193
             cd_ray ray;
