@@ -329,7 +329,8 @@ class DeformableBatch:
         self.tP, self.tF, h = heightfield(terrain_n, terrain_size, 5.0, seed=seed + 1)
         # world placement: uniform scale 1-2, on the terrain, random heading, half sunk
         self.scale = rng.uniform(1.0, 2.0, n_meshes)
-        xy = rng.uniform(10.0, terrain_size - 10.0, size=(n_meshes, 2))
+        edge = 10.0 if terrain_size >= 20.0 else 0.25 * terrain_size
+        xy = rng.uniform(edge, terrain_size - edge, size=(n_meshes, 2))
         gi = np.clip(np.rint(xy / terrain_size * (terrain_n - 1)).astype(int), 0, terrain_n - 1)
         z = h[gi[:, 0], gi[:, 1]]
         self.world_t = np.concatenate([xy, z[:, None]], 1)
