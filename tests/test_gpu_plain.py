@@ -68,6 +68,13 @@ def test_tree_build_matches_oracle(gpu, gpu_l1, orc, L):
         assert np.array_equal(got["perm"], want["perm"]), name
 
 
+def _slack_is(slack, tree, what):
+    """A mesh's slack is the oracle's but for the rounding of its formula and one step up to a float: never less, or
+    the batched traversal could reject a box that touches, and not much more."""
+    want = float(tree.slack)
+    assert want * (1 - 1e-6) <= slack <= want * (1 + 1e-5) + 1e-30, (slack, want, what)
+
+
 def _tiled_mesh(kind, n):
     """n triangles whose coordinate sums are of one kind: order of magnitude
     changes, half-way roundings and zeros of a running double sum."""
@@ -100,7 +107,7 @@ def test_tree_build_tiled_nodes(gpu, orc, kind):
         assert got["obbs"].tobytes() == want["obbs"].tobytes(), n
         assert np.array_equal(got["links"], want["links"]), n
         assert np.array_equal(got["perm"], want["perm"]), n
-        assert gpu.mesh_info(mid)["slack"] >= np.float32(tree.slack) * (1 - 1e-6), n
+        _slack_is(gpu.mesh_info(mid)["slack"], tree, n)
 
 
 def test_tree_build_keeps_its_buffers():
@@ -138,6 +145,7 @@ def test_tree_build_many_small_meshes(gpu, orc):
         want, got = tree.export(), gpu.export_tree(ids[k])
         for name in ("root", "obbs", "links", "perm"):
             assert np.asarray(got[name]).tobytes() == np.asarray(want[name]).tobytes(), (k, len(meshes[k]), name)
+        _slack_is(gpu.mesh_info(ids[k])["slack"], tree, (k, len(meshes[k])))
         assert gpu.mesh_info(ids[k])["radius"] >= np.sqrt((meshes[k].reshape(-1, 3).astype(np.float64) ** 2)
                                                           .sum(1).max(initial=0.0)) * (1 - 1e-7)
 
@@ -162,20 +170,31 @@ def test_tree_build_hand_derived_splits(gpu_l1, orc):
             assert got["obbs"].tobytes() == want["obbs"].tobytes(), name
 
 
-def test_tree_build_levels_wider_than_one_launch(gpu_l1, orc):
-    """A mesh whose deepest levels hold more nodes than one level launch has
-    workgroups (65,536), so the launch strides over them, and deeper than one
-    batch of level launches: bit-identical to the oracle's tree."""
+@pytest.mark.parametrize("freq", [32, 128])
+def test_tree_build_levels_wider_than_one_launch(gpu_l1, orc, freq):
+    """Meshes whose deepest levels hold more nodes than a level launch has
+    workgroups (8,192), so the launches stride over them, and deeper than one
+    batch of level launches.  Over 20,480 triangles such levels stay below
+    32,768 nodes and are k_level's; over 327,680 the wider ones go to
+    k_level_tiny, but for their nodes of more than 16 triangles, with one mesh
+    to a wavefront.  Bit-identical to the oracle's tree, and its slack."""
     rng = np.random.default_rng(5)
-    tri = scenes.displaced_icosphere(128, 0.1, rng)
+    tri = scenes.displaced_icosphere(freq, 0.1, rng)
     case(f"tree build, one mesh of {len(tri)} triangles, leaf size 1")
-    got = gpu_l1.export_tree(gpu_l1.register_soups([tri])[0])
-    want = orc.tree(tri, 1).export()
-    assert len(got["links"]) > 2 * 65536
+    mid = gpu_l1.register_soups([tri])[0]
+    got = gpu_l1.export_tree(mid)
+    tree = orc.tree(tri, 1)
+    want = tree.export()
+    links, level, width = got["links"], np.array([0]), []
+    while len(level):  # nodes per level, leaves included: twice the internal nodes of the level above
+        width.append(2 * len(level))
+        level = links[level][:, :2][links[level][:, 2:] == 0]
+    assert max(width) > 8192 and (max(width) < 32768) == (freq == 32)
     assert got["root"].tobytes() == want["root"].tobytes()
     assert got["obbs"].tobytes() == want["obbs"].tobytes()
     assert np.array_equal(got["links"], want["links"])
     assert np.array_equal(got["perm"], want["perm"])
+    _slack_is(gpu_l1.mesh_info(mid)["slack"], tree, freq)
 
 
 @pytest.mark.parametrize("L", [4, 1])
