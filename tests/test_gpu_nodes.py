@@ -167,3 +167,22 @@ def test_node_globals_time_grows_with_the_nodes():
                 t.append((time.perf_counter() - t0) * 1e3)
             ms.append(min(t))
     assert ms[1] < 8 * ms[0], ms
+
+
+@pytest.mark.parametrize("children_first", [False, True])
+@pytest.mark.parametrize("depth", [30, 31, 32, 33, 64, 255, 256, 257])
+def test_node_globals_chains(gpu, orc, depth, children_first):
+    """One straight chain: around the 32 ancestors a lane keeps at hand, and at the deepest that is accepted (256)."""
+    case(f"node globals, a chain of depth {depth}, {'children' if children_first else 'parents'} first")
+    n = depth + 1
+    rng = np.random.default_rng(depth)
+    trs, _ = _forest_parents_first(n, depth)
+    trs[:, 0:3] = rng.uniform(0.97, 1.03, (n, 3))
+    par = np.arange(n, dtype=np.uint32) - np.uint32(1)  # the first is the root: 0xFFFFFFFF
+    if children_first:
+        trs, par = trs[::-1].copy(), np.r_[np.arange(1, n), 0xFFFFFFFF].astype(np.uint32)
+    if depth > 256:
+        with pytest.raises(CollideError, match="deeper than 256"):
+            gpu.node_globals(_records(trs, par))
+        return
+    assert gpu.node_globals(_records(trs, par)).tobytes() == orc.node_globals(trs, par).tobytes()
