@@ -86,6 +86,40 @@ def test_response_scene_frames(gpu, orc):
     assert total > 10 and shot > 0
 
 
+@pytest.mark.parametrize("scale", [(1, 1, 1e-2), (1, 1, 1e-3), (1e3, 1e3, 1), (1e5, 1e5, 1), (1e3, 1, 1), (1e5, 1, 1),
+                                   (1e5, 1e5, 1e5), (1e5, 1e3, 1)])
+def test_response_near_degenerate_boxes(gpu, orc, scale):
+    """Spheres drawn out to plates and needles, and huge: boxes whose sides differ by up to 1e5, where the walk's
+    bound on a box test's rounding (from the slab records, for orthogonal sides) must still cover it.  Too small a
+    bound loses hits; the oracle runs the reference's own test on every box."""
+    case(f"response, spheres scaled by {scale}")
+    P, F = scenes.icosphere(6)
+    rng = np.random.default_rng(17)
+    P = P * (1.0 + rng.uniform(-0.02, 0.02, (len(P), 1)))
+    R = scenes.quat_to_mat3(scenes.random_quaternions(rng, 1))[0]
+    turn = np.array([[0.8, -0.6, 0.0], [0.6, 0.8, 0.0], [0.0, 0.0, 1.0]])
+    soups = [((P * np.array(scale)) @ R.T).astype(np.float32)[F].reshape(-1, 9),
+             (((P @ turn.T) * np.array(scale)) @ R.T).astype(np.float32)[F].reshape(-1, 9)]
+    ids = gpu.register_soups(soups)
+    trees = [orc.tree(m, 4) for m in soups]
+    shot = 0
+    for k in range(6):
+        d = R @ (rng.uniform(0.2, 0.9, 3) * np.array(scale))
+        e = np.zeros(2, ENTITY_DTYPE)
+        e["current"] = [scenes.identity16(), _tmat(*d)]
+        e["previous"] = [scenes.identity16(), _tmat(*(1.5 * d))]
+        e["mesh_id"] = ids
+        e["should_callback"] = 1
+        gpu.frame(e, MODE_PLAIN)
+        gpu.uncollide_rays()
+        got = gpu.shoot_rays()
+        want_ids, want_d, _ = orc.shoot_frame(trees, [0, 1], e["current"], e["previous"], e["should_callback"], COS_START,
+                                              COS_FINISH, np.float32(1.01))
+        _compare(got, want_ids, want_d)
+        shot += int(got["shot"].sum())
+    assert shot > 0
+
+
 def test_response_batched_mode_invariants(gpu):
     """After an exact-semantics frame the response has the same shape: a
     push apart along the centre line, shared by the entity that moved."""
