@@ -1624,15 +1624,15 @@ int rays_impl(cd_ctx* ctx, cd_pair_rays* pairs, uint32_t pair_cap, uint32_t* n_p
         // both orders at once per query, unless a query had more contacts than that ranks
         uint32_t bits[3];
         contact_field_bits(ctx, nq, bits);
-        const bool per_query = !ctx->contacts_sorted && !ctx->rays_radix && seg_order_fits(bits[1]);
+        const bool per_query = !ctx->contacts_sorted && !ctx->rays_radix;
         HCK(ctx, launch_fill_u32(tot, RAY_TOT_WORDS, 0u, st));
         if (per_query) {
             HCK(ctx, ctx->d_work[W_SEGQ].ensure(size_t(seg_order_words(nq)) * sizeof(uint32_t)));
             HCK(ctx, ctx->d_work[W_CSEG].ensure(size_t(nc) * sizeof(cd_contact)));
             uint32_t* qw = ctx->d_work[W_SEGQ].as<uint32_t>();
             HCK(ctx, launch_fill_u32(qw, nq, 0u, st));
-            HCK(ctx, launch_seg_order(ctx->d_contacts.as<cd_contact>(), nc, nullptr, nq, nullptr, &tot[DC_BIGSEG], qw,
-                                      ctx->d_work[W_CSEG].as<cd_contact>(), ctx->d_work[W_CSORT].as<cd_contact>(),
+            HCK(ctx, launch_seg_order(ctx->d_contacts.as<cd_contact>(), bits[1], nc, nullptr, nq, nullptr, &tot[DC_BIGSEG],
+                                      qw, ctx->d_work[W_CSEG].as<cd_contact>(), ctx->d_work[W_CSORT].as<cd_contact>(),
                                       ctx->d_work[W_V0].as<uint32_t>(), st));
         } else if (!ctx->contacts_sorted) {
             HCK(ctx, launch_sort_contacts(ctx->d_contacts.as<cd_contact>(), nc, ctx->d_work[W_CSORT].as<cd_contact>(),
@@ -1826,17 +1826,17 @@ int enqueue_step(cd_ctx* ctx, const StepArgs& a) {
     int rc = enqueue_batched(ctx, P, a.t, a.timed, a.ref);
     if (rc) return rc;
     const uint64_t ccap = std::min<uint64_t>(C, ctx->contact_cap);
+    uint32_t bits[3];
+    contact_field_bits(ctx, P, bits);
     if (a.radix) {
         HCK(ctx, launch_step_contacts(dev_counters(ctx), ccap, dc, st));
-        uint32_t bits[3];
-        contact_field_bits(ctx, P, bits);
         HCK(ctx, launch_sort_contacts(ctx->d_contacts.as<cd_contact>(), C, ctx->d_work[W_CSORT].as<cd_contact>(), bits,
                                       k0, v0, k1, v1, table, st, &dc[DC_NC]));
     } else {
         uint32_t* qw3 = ctx->d_work[W_SEGQ].as<uint32_t>();
         HCK(ctx, launch_step_contacts(dev_counters(ctx), ccap, dc, st, qw3, P));
-        HCK(ctx, launch_seg_order(ctx->d_contacts.as<cd_contact>(), C, &dc[DC_NC], P, &dc[DC_NQ], &dc[DC_BIGSEG], qw3,
-                                  ctx->d_work[W_CSEG].as<cd_contact>(),
+        HCK(ctx, launch_seg_order(ctx->d_contacts.as<cd_contact>(), bits[1], C, &dc[DC_NC], P, &dc[DC_NQ],
+                                  &dc[DC_BIGSEG], qw3, ctx->d_work[W_CSEG].as<cd_contact>(),
                                   ctx->d_work[W_CSORT].as<cd_contact>(), v0, st));
     }
     const StepLayout L(P, a.shoot);
@@ -1940,9 +1940,7 @@ int device_run(cd_ctx* ctx, const cd_entity* ents, uint32_t n, bool ref, bool sh
         a.np = ctx->step_np_cap;
         a.nc = ctx->step_nc_cap;
         a.rays = ctx->step_ray_cap;
-        uint32_t bits[3];
-        contact_field_bits(ctx, a.np, bits);
-        a.radix = ctx->step_radix || !seg_order_fits(bits[1]);
+        a.radix = ctx->step_radix;
         a.t = effective_tuning(ctx, a.np);
         uint64_t fcap = 0;
         int rc = ensure_step(ctx, a, &fcap);

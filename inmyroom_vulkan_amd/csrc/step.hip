@@ -59,7 +59,12 @@ __global__ __launch_bounds__(1024) void k_step_contacts(const RunCounters* __res
 constexpr uint32_t SEG_MAX = 4096, SEG_THREADS = 1024;
 constexpr uint32_t SEG_SMALL = 256;
 constexpr uint32_t SEG_GRID = 1024;   // workgroups of the larger pairs' launch at most
-constexpr uint32_t SEG_TRI_BITS = 25, SEG_POS_BITS = 13;  // a key: both triangles, and the contact's place
+// A key: both triangles, and the contact's place.  Where a mesh has more than
+// 2^25 triangles (WIDE) both take 32 bits each, and the places lie beside the
+// keys: 96 KB of LDS a workgroup instead of 80, for calls that would else need
+// the radix sorts (a frame of 63 pairs on a 34M-triangle terrain: 0.49 against
+// 0.62 ms with those).
+constexpr uint32_t SEG_TRI_BITS = 25, SEG_POS_BITS = 13;
 static_assert(2 * SEG_TRI_BITS + SEG_POS_BITS < 64 && SEG_MAX < (1u << SEG_POS_BITS), "key fields");
 
 // Slot of each lane's contact among its pair's (base + rank among the
@@ -148,10 +153,18 @@ __global__ __launch_bounds__(256) void k_seg_scatter(const cd_contact* __restric
 // are merged into runs of 2 L, every key by a binary search of the run next
 // to it (keys are distinct): each level's searches of all of a thread's keys
 // in both orders are in flight together, and a level costs two barriers.
-template <uint32_t THREADS, uint32_t CAP>
+template <uint32_t CAP, bool WIDE>
+struct SegShared {
+    unsigned long long key[2][CAP];
+    uint32_t place[CAP];
+    uint16_t pos[WIDE ? 2 : 1][WIDE ? CAP : 1];
+};
+template <uint32_t THREADS, uint32_t CAP, bool WIDE>
 __device__ __forceinline__ void seg_rank(const cd_contact* __restrict__ seg, uint32_t base, uint32_t n,
-                                         unsigned long long (*key)[CAP], uint32_t* place,
-                                         cd_contact* __restrict__ sorted, uint32_t* __restrict__ order_b) {
+                                         SegShared<CAP, WIDE>& S, cd_contact* __restrict__ sorted,
+                                         uint32_t* __restrict__ order_b) {
+    unsigned long long(*const key)[CAP] = S.key;
+    uint32_t* const place = S.place;
     constexpr uint32_t E = CAP / THREADS;
     const uint32_t tid = threadIdx.x;
 #pragma unroll
@@ -159,19 +172,30 @@ __device__ __forceinline__ void seg_rank(const cd_contact* __restrict__ seg, uin
         const uint32_t i = e * THREADS + tid;
         if (i < n) {
             const unsigned long long a = seg[base + i].tri_a, b = seg[base + i].tri_b;
-            key[0][i] = (((a << SEG_TRI_BITS) | b) << SEG_POS_BITS) | i;
-            key[1][i] = (((b << SEG_TRI_BITS) | a) << SEG_POS_BITS) | i;
+            if (WIDE) {
+                key[0][i] = (a << 32) | b;
+                key[1][i] = (b << 32) | a;
+                S.pos[0][i] = S.pos[WIDE][i] = uint16_t(i);
+            } else {
+                key[0][i] = (((a << SEG_TRI_BITS) | b) << SEG_POS_BITS) | i;
+                key[1][i] = (((b << SEG_TRI_BITS) | a) << SEG_POS_BITS) | i;
+            }
         }
     }
     __syncthreads();
     for (uint32_t lg = 0, L = 1; L < n; ++lg, L <<= 1) {
         unsigned long long v[2][E];
         uint32_t s0[E], len[E], lo[2][E];
+        uint16_t p[2][E];
 #pragma unroll
         for (uint32_t e = 0; e < E; ++e) {
             const uint32_t i = min(e * THREADS + tid, n - 1);
             v[0][e] = key[0][i];
             v[1][e] = key[1][i];
+            if (WIDE) {
+                p[0][e] = S.pos[0][i];
+                p[1][e] = S.pos[WIDE][i];
+            }
             s0[e] = min(((i >> lg) ^ 1u) << lg, n);  // the run next to key i's
             len[e] = min(L, n - s0[e]);
             lo[0][e] = lo[1][e] = 0;
@@ -196,17 +220,23 @@ __device__ __forceinline__ void seg_rank(const cd_contact* __restrict__ seg, uin
                 const uint32_t at = (((i >> lg) & ~1u) << lg) + (i & (L - 1));
                 key[0][at + lo[0][e]] = v[0][e];
                 key[1][at + lo[1][e]] = v[1][e];
+                if (WIDE) {
+                    S.pos[0][at + lo[0][e]] = p[0][e];
+                    S.pos[WIDE][at + lo[1][e]] = p[1][e];
+                }
             }
         }
         __syncthreads();
     }
-    // slot r of the sorted array holds contact (key & mask); the second order lists those slots
-    constexpr uint32_t MASK = (1u << SEG_POS_BITS) - 1u;
+    // slot r of the sorted array holds the contact at key r's place; the second order lists those slots
+    auto placed = [&](int o, uint32_t r) -> uint32_t {
+        return WIDE ? S.pos[o * WIDE][r] : uint32_t(key[o][r]) & ((1u << SEG_POS_BITS) - 1u);
+    };
 #pragma unroll
     for (uint32_t e = 0; e < E; ++e) {
         const uint32_t r = e * THREADS + tid;
         if (r < n) {
-            const uint32_t i = uint32_t(key[0][r]) & MASK;
+            const uint32_t i = placed(0, r);
             place[i] = r;
             sorted[base + r] = seg[base + i];
         }
@@ -215,32 +245,32 @@ __device__ __forceinline__ void seg_rank(const cd_contact* __restrict__ seg, uin
 #pragma unroll
     for (uint32_t e = 0; e < E; ++e) {
         const uint32_t r = e * THREADS + tid;
-        if (r < n) order_b[base + r] = base + place[uint32_t(key[1][r]) & MASK];
+        if (r < n) order_b[base + r] = base + place[placed(1, r)];
     }
 }
 
+template <bool WIDE>
 __global__ __launch_bounds__(SEG_SMALL) void k_seg_sort_small(const cd_contact* __restrict__ seg,
                                                        const uint32_t* __restrict__ qoff,
                                                        const uint32_t* __restrict__ qcnt,
                                                        const uint32_t* __restrict__ nq_dev, uint32_t cap,
                                                        cd_contact* __restrict__ sorted, uint32_t* __restrict__ order_b) {
-    __shared__ unsigned long long s_key[2][SEG_SMALL];
-    __shared__ uint32_t s_place[SEG_SMALL];
+    __shared__ SegShared<SEG_SMALL, WIDE> S;
     const uint32_t q = blockIdx.x;
     if (q >= count_of(cap, nq_dev)) return;
     const uint32_t n = qcnt[q];
     if (n == 0 || n > SEG_SMALL) return;
-    seg_rank<SEG_SMALL, SEG_SMALL>(seg, qoff[q], n, s_key, s_place, sorted, order_b);
+    seg_rank<SEG_SMALL, SEG_SMALL, WIDE>(seg, qoff[q], n, S, sorted, order_b);
 }
 
+template <bool WIDE>
 __global__ __launch_bounds__(SEG_THREADS) void k_seg_sort(const cd_contact* __restrict__ seg,
                                                           const uint32_t* __restrict__ qoff,
                                                           const uint32_t* __restrict__ qcnt,
                                                           const uint32_t* __restrict__ large,
                                                           cd_contact* __restrict__ sorted,
                                                           uint32_t* __restrict__ order_b) {
-    __shared__ unsigned long long s_key[2][SEG_MAX];
-    __shared__ uint32_t s_place[SEG_MAX];
+    __shared__ SegShared<SEG_MAX, WIDE> S;
     for (uint32_t k = blockIdx.x; k < large[0]; k += gridDim.x) {
         const uint32_t q = large[1 + k], n = qcnt[q];
         if (n > SEG_MAX) {  // flagged: in any order, so that what follows reads contacts
@@ -250,7 +280,7 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg_sort(const cd_contact* __re
             }
             continue;
         }
-        seg_rank<SEG_THREADS, SEG_MAX>(seg, qoff[q], n, s_key, s_place, sorted, order_b);
+        seg_rank<SEG_THREADS, SEG_MAX, WIDE>(seg, qoff[q], n, S, sorted, order_b);
         __syncthreads();  // the next pair reuses the LDS
     }
 }
@@ -308,8 +338,7 @@ hipError_t launch_step_contacts(const RunCounters* ctr, uint64_t cap, uint32_t* 
     return hipGetLastError();
 }
 uint32_t seg_order_words(uint32_t np_cap) { return 4 * np_cap + 1; }
-bool seg_order_fits(uint32_t tri_bits) { return tri_bits <= SEG_TRI_BITS; }
-hipError_t launch_seg_order(const cd_contact* c, uint32_t nc_cap, const uint32_t* nc_dev, uint32_t np_cap,
+hipError_t launch_seg_order(const cd_contact* c, uint32_t tri_bits, uint32_t nc_cap, const uint32_t* nc_dev, uint32_t np_cap,
                             const uint32_t* np_dev, uint32_t* flag, uint32_t* work, cd_contact* seg, cd_contact* sorted,
                             uint32_t* order_b, hipStream_t st) {
     uint32_t* qcnt = work;
@@ -320,11 +349,19 @@ hipError_t launch_seg_order(const cd_contact* c, uint32_t nc_cap, const uint32_t
     hipLaunchKernelGGL(k_seg_count, gc, dim3(256), 0, st, c, nc_cap, nc_dev, qcnt);
     hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, st, qcnt, np_cap, np_dev, qoff, qfill, large, flag);
     hipLaunchKernelGGL(k_seg_scatter, gc, dim3(256), 0, st, c, nc_cap, nc_dev, qfill, seg);
-    hipLaunchKernelGGL(k_seg_sort_small, dim3(std::max(np_cap, 1u)), dim3(SEG_SMALL), 0, st, seg, qoff, qcnt, np_dev, np_cap,
-                       sorted, order_b);
     // no more pairs than contacts / SEG_SMALL are large
-    const uint32_t gl = std::min(std::min(np_cap, nc_cap / SEG_SMALL), SEG_GRID);
-    if (gl) hipLaunchKernelGGL(k_seg_sort, dim3(gl), dim3(SEG_THREADS), 0, st, seg, qoff, qcnt, large, sorted, order_b);
+    const dim3 gs(std::max(np_cap, 1u)), gl(std::min(std::min(np_cap, nc_cap / SEG_SMALL), SEG_GRID));
+    if (tri_bits > SEG_TRI_BITS) {
+        hipLaunchKernelGGL(k_seg_sort_small<true>, gs, dim3(SEG_SMALL), 0, st, seg, qoff, qcnt, np_dev, np_cap, sorted,
+                           order_b);
+        if (gl.x)
+            hipLaunchKernelGGL(k_seg_sort<true>, gl, dim3(SEG_THREADS), 0, st, seg, qoff, qcnt, large, sorted, order_b);
+    } else {
+        hipLaunchKernelGGL(k_seg_sort_small<false>, gs, dim3(SEG_SMALL), 0, st, seg, qoff, qcnt, np_dev, np_cap, sorted,
+                           order_b);
+        if (gl.x)
+            hipLaunchKernelGGL(k_seg_sort<false>, gl, dim3(SEG_THREADS), 0, st, seg, qoff, qcnt, large, sorted, order_b);
+    }
     return hipGetLastError();
 }
 hipError_t launch_pair_begins(const uint32_t* qw, uint32_t stride, const uint32_t* dc, uint32_t* pbegin, hipStream_t st) {

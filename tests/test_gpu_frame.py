@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 from conftest import case
-from inmyroom_vulkan_amd import ENTITY_DTYPE, MODE_BATCHED, MODE_PLAIN, scenes
+from inmyroom_vulkan_amd import ENTITY_DTYPE, MODE_BATCHED, MODE_PLAIN, MODE_REFERENCE, Collider, scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -244,3 +244,37 @@ def test_broad_phase_ends_the_last_run(gpu):
     for call in (gpu.uncollide_rays, gpu.shoot_rays):
         with pytest.raises(CollideError):
             call()
+
+
+def test_frame_on_a_mesh_beyond_25_bit_triangles():
+    """A terrain of 42,301,602 triangles: the per-pair contact order's keys take 32 bits a triangle there.  Small
+    spheres over all of it, one pair with more contacts than a small workgroup orders; the frame's contacts are in the
+    plain frame's order (radix sorts), and so are its rays."""
+    n = 4600
+    x = np.linspace(0, 100, n, dtype=np.float32)
+    P = np.empty((n, n, 3), np.float32)
+    P[..., 0], P[..., 1] = x[:, None], x[None, :]
+    P[..., 2] = np.sin(x)[:, None] * np.cos(x)[None, :]
+    i = np.arange(n * (n - 1), dtype=np.uint32).reshape(n - 1, n)[:, :-1].ravel()
+    F = np.concatenate([np.stack([i, i + n, i + 1], 1), np.stack([i + 1, i + n, i + n + 1], 1)])
+    assert len(F) > 1 << 25
+    case(f"frame on a terrain of {len(F)} triangles")
+    S, G = scenes.icosphere(8)
+    with Collider(leaf_max=4) as gpu:
+        terrain = gpu.register_mesh(P.reshape(-1, 3), F)
+        ball = gpu.register_mesh((0.05 * S).astype(np.float32), G)
+        xy = np.random.default_rng(1).uniform(0.5, 99.5, (40, 2))
+        e = np.zeros(len(xy) + 1, ENTITY_DTYPE)
+        e["current"] = scenes.identity16()
+        e["current"][1:, 12:14] = xy
+        e["current"][1:, 14] = np.sin(xy[:, 0]) * np.cos(xy[:, 1])
+        e["previous"] = e["current"]
+        e["mesh_id"] = [terrain] + [ball] * len(xy)
+        e["should_callback"] = 1
+        pairs, cons = gpu.frame(e, MODE_REFERENCE)
+        _, rays = gpu.uncollide_rays()
+        want_pairs, want = gpu.frame(e, MODE_PLAIN)
+        _, want_rays = gpu.uncollide_rays()
+        assert int(pairs["contact_count"].max()) > 256 and max(want["tri_a"].max(), want["tri_b"].max()) > 1 << 25
+        assert pairs.tobytes() == want_pairs.tobytes() and cons.tobytes() == want.tobytes()
+        assert rays.tobytes() == want_rays.tobytes()
