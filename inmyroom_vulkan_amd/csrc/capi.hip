@@ -241,9 +241,11 @@ void contact_field_bits(const cd_ctx* ctx, uint32_t nq, uint32_t bits[3]) {
 // Enqueue the whole batched pipeline on the stream (no host synchronisation
 // inside, so it can be captured in a graph).
 uint64_t frontier_cap(const cd_ctx* ctx, uint32_t nq, uint32_t L) {
-    // worst case nq * 2^L, capped; a level that overflows sets an error bit and the run is repeated larger
+    // worst case nq * 2^L, capped; a level that overflows sets an error bit and the run is repeated larger.  The first
+    // frontier holds a pair of roots per query, whatever the cap.
     const uint64_t worst = (L >= 40) ? (uint64_t(1) << 40) : (uint64_t(std::max(nq, 1u)) << L);
-    return std::max<uint64_t>(64, std::min<uint64_t>(worst, std::max<uint64_t>(ctx->frontier_cap, 1u << 20)));
+    return std::max<uint64_t>(std::max(nq, 64u),
+                              std::min<uint64_t>(worst, std::max<uint64_t>(ctx->frontier_cap, 1u << 20)));
 }
 
 // nq: the capacity the launch geometry is built for; the count itself is in d_nq

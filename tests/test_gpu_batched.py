@@ -11,7 +11,7 @@ import pytest
 from conftest import case, golden
 from contacts_check import (MIN_SIN, SEG_TOL, TreePositions, assert_same_keys, check_batched_geometry,
                             corners_from_trees, crossing_sin, sort_contacts)
-from inmyroom_vulkan_amd import MODE_BATCHED, MODE_PLAIN, scenes
+from inmyroom_vulkan_amd import MODE_BATCHED, MODE_PLAIN, MODE_REFERENCE, Collider, scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -205,3 +205,23 @@ def test_batched_graph_replays_match_eager(gpu):
             gpu.stage(q)
     finally:
         gpu.set_tuning()
+
+
+def test_batch_of_more_queries_than_the_first_frontier_held():
+    """1,100,000 queries: the traversal's first frontier holds a pair of roots for each, also beyond 2^20 entries, the
+    capacity it starts from.  A few hundred touch, the last ones among them; the plain path's contacts."""
+    nq = 1_100_000
+    mesh = scenes.unit_icosphere_soup(2).astype(np.float32)
+    near = np.unique(np.r_[np.arange(0, nq, 5003), np.arange(nq - 50, nq)])
+    rel = np.tile(scenes.identity16(), (nq, 1)).astype(np.float32)
+    rel[:, 12] = 9.0
+    rel[near, 12] = 1.7
+    case(f"{nq} queries, {len(near)} touching")
+    with Collider(leaf_max=4) as gpu:
+        mid = gpu.register_soups([mesh])[0]
+        gpu.stage(gpu.make_queries(mid, mid, rel))
+        n = {m: gpu.run_staged(m) for m in (MODE_PLAIN, MODE_REFERENCE, MODE_BATCHED)}
+        pairs, rays = gpu.uncollide_rays()
+    assert n[MODE_REFERENCE] == n[MODE_PLAIN] > 0
+    assert n[MODE_BATCHED] > 0 and n[MODE_BATCHED] % len(near) == 0  # the same pose: the same contacts each
+    assert np.array_equal(pairs["query"], near) and len(rays) > 0
