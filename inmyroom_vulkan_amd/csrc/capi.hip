@@ -1629,7 +1629,7 @@ int rays_impl(cd_ctx* ctx, cd_pair_rays* pairs, uint32_t pair_cap, uint32_t* n_p
         const bool per_query = !ctx->contacts_sorted && !ctx->rays_radix;
         HCK(ctx, launch_fill_u32(tot, RAY_TOT_WORDS, 0u, st));
         if (per_query) {
-            HCK(ctx, ctx->d_work[W_SEGQ].ensure(size_t(seg_order_words(nq)) * sizeof(uint32_t)));
+            HCK(ctx, ctx->d_work[W_SEGQ].ensure(seg_order_words(nq) * sizeof(uint32_t)));
             HCK(ctx, ctx->d_work[W_CSEG].ensure(size_t(nc) * sizeof(cd_contact)));
             uint32_t* qw = ctx->d_work[W_SEGQ].as<uint32_t>();
             HCK(ctx, launch_fill_u32(qw, nq, 0u, st));
@@ -1776,7 +1776,7 @@ int ensure_step(cd_ctx* ctx, const StepArgs& a, uint64_t* fcap) {
     HCK(ctx, sort_table(ctx, std::max(std::max(n, P), C), &table));
     HCK(ctx, ctx->d_work[W_SCTR].ensure(sizeof(RunCounters)));
     HCK(ctx, ctx->d_work[W_STEPC].ensure(DC_WORDS * sizeof(uint32_t)));
-    HCK(ctx, ctx->d_work[W_SEGQ].ensure(size_t(seg_order_words(P)) * sizeof(uint32_t)));
+    HCK(ctx, ctx->d_work[W_SEGQ].ensure(seg_order_words(P) * sizeof(uint32_t)));
     HCK(ctx, ctx->d_work[W_CSEG].ensure(size_t(C) * sizeof(cd_contact)));
     if (a.shoot) {
         HCK(ctx, ctx->d_work[W_PIDS].ensure(2 * size_t(P) * sizeof(uint32_t)));

@@ -193,7 +193,7 @@ hipError_t launch_step_contacts(const RunCounters* ctr, uint64_t cap, uint32_t* 
 // seg nc_cap contacts of scratch.  *flag is set when a pair has more contacts
 // than one workgroup ranks, and the order is then incomplete.  tri_bits: bits
 // that hold every triangle index.
-uint32_t seg_order_words(uint32_t np_cap);
+size_t seg_order_words(uint32_t np_cap);
 hipError_t launch_seg_order(const cd_contact* c, uint32_t tri_bits, uint32_t nc_cap, const uint32_t* nc_dev, uint32_t np_cap,
                             const uint32_t* np_dev, uint32_t* flag, uint32_t* work, cd_contact* seg, cd_contact* sorted,
                             uint32_t* order_b, hipStream_t st);

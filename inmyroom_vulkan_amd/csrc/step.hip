@@ -59,6 +59,7 @@ __global__ __launch_bounds__(1024) void k_step_contacts(const RunCounters* __res
 constexpr uint32_t SEG_MAX = 4096, SEG_THREADS = 1024;
 constexpr uint32_t SEG_SMALL = 256;
 constexpr uint32_t SEG_GRID = 1024;   // workgroups of the larger pairs' launch at most
+constexpr uint32_t SEG_SMALL_GRID = 1u << 20;  // of the small ones': a launch takes fewer than 2^32 threads
 // A key: both triangles, and the contact's place.  Where a mesh has more than
 // 2^25 triangles (WIDE) both take 32 bits each, and the places lie beside the
 // keys: 96 KB of LDS a workgroup instead of 80, for calls that would else need
@@ -256,11 +257,13 @@ __global__ __launch_bounds__(SEG_SMALL) void k_seg_sort_small(const cd_contact* 
                                                        const uint32_t* __restrict__ nq_dev, uint32_t cap,
                                                        cd_contact* __restrict__ sorted, uint32_t* __restrict__ order_b) {
     __shared__ SegShared<SEG_SMALL, WIDE> S;
-    const uint32_t q = blockIdx.x;
-    if (q >= count_of(cap, nq_dev)) return;
-    const uint32_t n = qcnt[q];
-    if (n == 0 || n > SEG_SMALL) return;
-    seg_rank<SEG_SMALL, SEG_SMALL, WIDE>(seg, qoff[q], n, S, sorted, order_b);
+    const uint32_t nq = count_of(cap, nq_dev);
+    for (uint32_t q = blockIdx.x; q < nq; q += gridDim.x) {
+        const uint32_t n = qcnt[q];
+        if (n == 0 || n > SEG_SMALL) continue;
+        seg_rank<SEG_SMALL, SEG_SMALL, WIDE>(seg, qoff[q], n, S, sorted, order_b);
+        __syncthreads();  // the next pair reuses the LDS
+    }
 }
 
 template <bool WIDE>
@@ -337,7 +340,7 @@ hipError_t launch_step_contacts(const RunCounters* ctr, uint64_t cap, uint32_t* 
     hipLaunchKernelGGL(k_step_contacts, dim3(1), dim3(1024), 0, st, ctr, cap, dc, qcnt, np);
     return hipGetLastError();
 }
-uint32_t seg_order_words(uint32_t np_cap) { return 4 * np_cap + 1; }
+size_t seg_order_words(uint32_t np_cap) { return 4 * size_t(np_cap) + 1; }
 hipError_t launch_seg_order(const cd_contact* c, uint32_t tri_bits, uint32_t nc_cap, const uint32_t* nc_dev, uint32_t np_cap,
                             const uint32_t* np_dev, uint32_t* flag, uint32_t* work, cd_contact* seg, cd_contact* sorted,
                             uint32_t* order_b, hipStream_t st) {
@@ -350,7 +353,8 @@ hipError_t launch_seg_order(const cd_contact* c, uint32_t tri_bits, uint32_t nc_
     hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, st, qcnt, np_cap, np_dev, qoff, qfill, large, flag);
     hipLaunchKernelGGL(k_seg_scatter, gc, dim3(256), 0, st, c, nc_cap, nc_dev, qfill, seg);
     // no more pairs than contacts / SEG_SMALL are large
-    const dim3 gs(std::max(np_cap, 1u)), gl(std::min(std::min(np_cap, nc_cap / SEG_SMALL), SEG_GRID));
+    const dim3 gs(std::min(std::max(np_cap, 1u), SEG_SMALL_GRID)),
+        gl(std::min(std::min(np_cap, nc_cap / SEG_SMALL), SEG_GRID));
     if (tri_bits > SEG_TRI_BITS) {
         hipLaunchKernelGGL(k_seg_sort_small<true>, gs, dim3(SEG_SMALL), 0, st, seg, qoff, qcnt, np_dev, np_cap, sorted,
                            order_b);
