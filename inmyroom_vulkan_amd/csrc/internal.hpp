@@ -318,9 +318,6 @@ struct cd_ctx {
     std::string scratch_err;               // why it could not be resolved
     hipGraphExec_t graph = nullptr;        // captured batched pipeline
     std::vector<uint64_t> graph_key;       // sizes, tuning and every device pointer the graph captured
-    // the frame and the scene step on the device: capacities (grown when a
-    // run exceeds one), their captured graphs and keys, and the pinned block
-    // their results land in
     // slab records of the ray shooting's box tests: two per internal node
     // (node arena order), one per mesh root; valid for a mesh until it is
     // refit
@@ -329,9 +326,13 @@ struct cd_ctx {
     // the tree build's work buffers, kept between builds that need at most
     // BUILD_KEEP bytes of them (a model load builds one document at a time)
     cdk::DevBuf build_scratch[cdk::BUILD_SCRATCH];
-    bool rays_radix = false;  // the same for cd_uncollide_rays after a query batch
+    // a query had more contacts than the per-query order ranks: later batches'
+    // contacts take the radix sorts; step_radix: the same for steps and frames
+    bool rays_radix = false, step_radix = false;
+    // the frame and the scene step on the device: capacities (grown when a
+    // run exceeds one), their captured graphs and keys, and the pinned block
+    // their results land in
     uint32_t step_np_cap = 0, step_nc_cap = 0, step_ray_cap = 0;
-    bool step_radix = false;  // a pair had more contacts than the per-pair order ranks: the radix sorts
     hipGraphExec_t step_graph = nullptr, frame_graph = nullptr;  // the whole step; cd_frame's part of it
     std::vector<uint64_t> step_key, frame_key;
     cdk::HostBuf h_step, h_ents;  // the run's result block; its entity records, staged for the graph's upload

@@ -3,7 +3,8 @@
 //  inMyRoom_vulkan/src/CollisionDetection/ShootUncollideRays.cpp:14-179;
 //  Ray::IntersectOBBtree, Ray.cpp:13-236; CollisionDetection.cpp:70-99, 143-150).
 //
-//  k_shoot    two lanes per uncollide ray.  Pass 1 shoots the ray at the
+//  k_shoot    two lanes per uncollide ray, or four where a call's rays fill no
+//             more than 16 to a wavefront (shootshape.hpp).  Pass 1 shoots the ray at the
 //             other entity's tree (closest hit, even lane); it succeeds when
 //             that hit is a back face reached before the ray re-enters its own
 //             tree (odd lane; the Hermann pass, :129-158).  On success the ray is reflected (origin
@@ -172,9 +173,11 @@ __device__ __forceinline__ RaySlab make_slab(const ChildRec& r) {
 // their own size beyond that, so both intervals differ from the crossing t by
 // at most e |r| (1 + rho) + rho |t|.  e is bounded by the 1-norms of the
 // normal, the centre and the half-sides; the latter's from the record: the
-// sides are orthogonal, so |u|_1 <= sqrt(3) |u| <= 3 h / |n|_1.  Written without branches: a node's two
-// tests are most of a step's instructions, with about one wavefront per SIMD,
-// and the exec-mask turns of the branches cost as much as the arithmetic.
+// sides are orthogonal, so |u|_1 <= sqrt(3) |u| <= 3 h / |n|_1 (0.1 more for
+// the rounding; tests/test_box_margin.py).  Written without branches: a
+// node's two tests are most of a step's instructions, with about one
+// wavefront per SIMD, and the exec-mask turns of the branches cost as much as
+// the arithmetic.
 enum : int { BOX_OUT = 0, BOX_IN = 1, BOX_NEAR = 2 };
 __device__ __forceinline__ int box_local(const LocalRay& R, const RaySlab& sl, float& tmin, float& tmax) {
     const float inf = __builtin_huge_valf();
