@@ -831,12 +831,14 @@ __global__ __launch_bounds__(64) void k_dfs(const uint3* __restrict__ tasks, con
             unsigned int base = 0;
             if (lane == 0) base = atomicAdd(ndump, n);
             base = __shfl(base, 0, 64);
-            if (base + n <= dump_cap && base + n >= base) {
-                for (uint32_t i = lane; i < size; i += 64) dump[base + i] = make_uint3(sq[i], sa[i], sb[i]);
-                for (uint32_t i = lane; i < nspill; i += 64) dump[base + size + i] = spill[i];
-            } else if (lane == 0) {
-                atomicOr(reinterpret_cast<unsigned int*>(&ctr->err), 2u);  // out of frontier room: rerun larger
-            }
+            // every entry below the capacity is written, also when the list runs out: the re-split reads them all
+            const uint64_t at = base;
+            for (uint32_t i = lane; i < size; i += 64)
+                if (at + i < dump_cap) dump[at + i] = make_uint3(sq[i], sa[i], sb[i]);
+            for (uint32_t i = lane; i < nspill; i += 64)
+                if (at + size + i < dump_cap) dump[at + size + i] = spill[i];
+            if (lane == 0 && at + n > dump_cap)  // out of room: rerun larger
+                atomicOr(reinterpret_cast<unsigned int*>(&ctr->err), 2u);
             size = 0;
             nspill = 0;
             break;
