@@ -109,8 +109,9 @@ hipError_t launch_sort_perm(const cd_contact* in, uint32_t n, int f_hi, int f_mi
 // response.hip
 // pbegin: per side (nq each) the first ray of every pair, non-decreasing;
 // stack_entries: the deepest tree the rays meet + 2; above RAY_STACK_ENTRIES
-// the stacks live in gstack, shoot_gstack_bytes(nrays, stack_entries) bytes; ctr->err gets bit 0 if a traversal stack would have overflowed,
-// ctr->sat the boxes tested and ctr->tritests the ray-triangle tests.
+// the stacks live in gstack, shoot_gstack_bytes(nrays, stack_entries) bytes;
+// ctr->err gets bit 0 if a traversal stack would have overflowed, ctr->sat
+// the boxes tested and ctr->tritests the ray-triangle tests.
 // stride: the per-side spacing of pbegin (0: nq); dc: the step's count block
 // (DC_*), from which the ray and pair counts are read when given, nrays and
 // nq being the capacities.
@@ -194,9 +195,9 @@ hipError_t launch_step_contacts(const RunCounters* ctr, uint64_t cap, uint32_t* 
 // than one workgroup ranks, and the order is then incomplete.  tri_bits: bits
 // that hold every triangle index.
 size_t seg_order_words(uint32_t np_cap);
-hipError_t launch_seg_order(const cd_contact* c, uint32_t tri_bits, uint32_t nc_cap, const uint32_t* nc_dev, uint32_t np_cap,
-                            const uint32_t* np_dev, uint32_t* flag, uint32_t* work, cd_contact* seg, cd_contact* sorted,
-                            uint32_t* order_b, hipStream_t st);
+hipError_t launch_seg_order(const cd_contact* c, uint32_t tri_bits, uint32_t nc_cap, const uint32_t* nc_dev,
+                            uint32_t np_cap, const uint32_t* np_dev, uint32_t* flag, uint32_t* work, cd_contact* seg,
+                            cd_contact* sorted, uint32_t* order_b, hipStream_t st);
 // pbegin[stride side + q]: the first ray of pair q on each side, from the
 // counts at qw + 2 stride side, for the dc[DC_NQ] pairs
 hipError_t launch_pair_begins(const uint32_t* qw, uint32_t stride, const uint32_t* dc, uint32_t* pbegin, hipStream_t st);

@@ -341,9 +341,9 @@ hipError_t launch_step_contacts(const RunCounters* ctr, uint64_t cap, uint32_t* 
     return hipGetLastError();
 }
 size_t seg_order_words(uint32_t np_cap) { return 4 * size_t(np_cap) + 1; }
-hipError_t launch_seg_order(const cd_contact* c, uint32_t tri_bits, uint32_t nc_cap, const uint32_t* nc_dev, uint32_t np_cap,
-                            const uint32_t* np_dev, uint32_t* flag, uint32_t* work, cd_contact* seg, cd_contact* sorted,
-                            uint32_t* order_b, hipStream_t st) {
+hipError_t launch_seg_order(const cd_contact* c, uint32_t tri_bits, uint32_t nc_cap, const uint32_t* nc_dev,
+                            uint32_t np_cap, const uint32_t* np_dev, uint32_t* flag, uint32_t* work, cd_contact* seg,
+                            cd_contact* sorted, uint32_t* order_b, hipStream_t st) {
     uint32_t* qcnt = work;
     uint32_t* qoff = work + np_cap;
     uint32_t* qfill = work + 2 * size_t(np_cap);
