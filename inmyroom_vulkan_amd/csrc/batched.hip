@@ -826,7 +826,17 @@ __global__ __launch_bounds__(64) void k_dfs(const uint3* __restrict__ tasks, con
             if (leave) break;
             continue;
         }
-        if (budget && wave_tests >= budget) {  // hand the rest of this stack on, then leave
+        // At its budget a wavefront hands the rest of its stack on and leaves,
+        // but not before every task is taken: with all of them gone the tasks
+        // left on the list would be nobody's.
+        bool spent = budget && wave_tests >= budget;
+        if (spent && !tasks_done) {
+            unsigned int taken = 0;
+            if (lane == 0) taken = coherent_read(head);
+            tasks_done = uint32_t(__shfl(taken, 0, 64)) >= ntasks;
+            spent = tasks_done;
+        }
+        if (spent) {
             const uint32_t n = size + nspill;
             unsigned int base = 0;
             if (lane == 0) base = atomicAdd(ndump, n);

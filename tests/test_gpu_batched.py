@@ -185,6 +185,24 @@ def test_batched_budgeted_pass_agrees(gpu, tuning):
         gpu.set_tuning()
 
 
+@pytest.mark.parametrize("handoff_pct", [50, 1])
+def test_batched_budgeted_pass_takes_every_task(handoff_pct):
+    """Far more tasks than the first launch's wavefronts can hold at once: none may reach its budget and leave while
+    tasks are left.  The budget also comes from a smaller batch before."""
+    mesh, rel = scenes.config1(4000, seed=3, freq=12)
+    case(f"budgeted pass over {len(rel)} poses, hand-over at {handoff_pct}%")
+    with Collider(leaf_max=4) as gpu:
+        mid = gpu.register_soups([mesh])[0]
+        want = {}
+        for n in (50, 4000):
+            gpu.stage(gpu.make_queries(mid, mid, rel[:n]))
+            want[n] = (gpu.run_staged(MODE_BATCHED), gpu.counters()["sat_tests"])
+        gpu.set_tuning(work_sharing=3, handoff_pct=handoff_pct, waves_per_cu=2)
+        for n in (50, 4000, 4000):
+            gpu.stage(gpu.make_queries(mid, mid, rel[:n]))
+            assert (gpu.run_staged(MODE_BATCHED), gpu.counters()["sat_tests"]) == want[n], n
+
+
 def test_batched_graph_replays_match_eager(gpu):
     soups, qa, qb, rel, _ = scenes.config3(96, seed=7, freq_cap=20)
     case("batched graph replays")
