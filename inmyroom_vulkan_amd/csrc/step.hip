@@ -62,9 +62,9 @@ constexpr uint32_t SEG_GRID = 1024;   // workgroups of the larger pairs' launch 
 constexpr uint32_t SEG_SMALL_GRID = 1u << 20;  // of the small ones': a launch takes fewer than 2^32 threads
 // A key: both triangles, and the contact's place.  Where a mesh has more than
 // 2^25 triangles (WIDE) both take 32 bits each, and the places lie beside the
-// keys: 96 KB of LDS a workgroup instead of 80, for calls that would else need
-// the radix sorts (a frame of 63 pairs on a 34M-triangle terrain: 0.49 against
-// 0.62 ms with those).
+// keys: 96 KB of LDS a workgroup (one to a CU) instead of 80 (two), against the
+// radix sorts such meshes would need (a frame of 63 pairs on a 34M-triangle
+// terrain: 0.49 against 0.62 ms).
 constexpr uint32_t SEG_TRI_BITS = 25, SEG_POS_BITS = 13;
 static_assert(2 * SEG_TRI_BITS + SEG_POS_BITS < 64 && SEG_MAX < (1u << SEG_POS_BITS), "key fields");
 
@@ -158,8 +158,14 @@ template <uint32_t CAP, bool WIDE>
 struct SegShared {
     unsigned long long key[2][CAP];
     uint32_t place[CAP];
-    uint16_t pos[WIDE ? 2 : 1][WIDE ? CAP : 1];
 };
+template <uint32_t CAP>
+struct SegShared<CAP, true> {
+    unsigned long long key[2][CAP];
+    uint32_t place[CAP];
+    uint16_t pos[2][CAP];
+};
+static_assert(sizeof(SegShared<SEG_MAX, false>) <= 80 * 1024, "two large workgroups share a CU's LDS");
 template <uint32_t THREADS, uint32_t CAP, bool WIDE>
 __device__ __forceinline__ void seg_rank(const cd_contact* __restrict__ seg, uint32_t base, uint32_t n,
                                          SegShared<CAP, WIDE>& S, cd_contact* __restrict__ sorted,
@@ -173,10 +179,10 @@ __device__ __forceinline__ void seg_rank(const cd_contact* __restrict__ seg, uin
         const uint32_t i = e * THREADS + tid;
         if (i < n) {
             const unsigned long long a = seg[base + i].tri_a, b = seg[base + i].tri_b;
-            if (WIDE) {
+            if constexpr (WIDE) {
                 key[0][i] = (a << 32) | b;
                 key[1][i] = (b << 32) | a;
-                S.pos[0][i] = S.pos[WIDE][i] = uint16_t(i);
+                S.pos[0][i] = S.pos[1][i] = uint16_t(i);
             } else {
                 key[0][i] = (((a << SEG_TRI_BITS) | b) << SEG_POS_BITS) | i;
                 key[1][i] = (((b << SEG_TRI_BITS) | a) << SEG_POS_BITS) | i;
@@ -193,9 +199,9 @@ __device__ __forceinline__ void seg_rank(const cd_contact* __restrict__ seg, uin
             const uint32_t i = min(e * THREADS + tid, n - 1);
             v[0][e] = key[0][i];
             v[1][e] = key[1][i];
-            if (WIDE) {
+            if constexpr (WIDE) {
                 p[0][e] = S.pos[0][i];
-                p[1][e] = S.pos[WIDE][i];
+                p[1][e] = S.pos[1][i];
             }
             s0[e] = min(((i >> lg) ^ 1u) << lg, n);  // the run next to key i's
             len[e] = min(L, n - s0[e]);
@@ -221,9 +227,9 @@ __device__ __forceinline__ void seg_rank(const cd_contact* __restrict__ seg, uin
                 const uint32_t at = (((i >> lg) & ~1u) << lg) + (i & (L - 1));
                 key[0][at + lo[0][e]] = v[0][e];
                 key[1][at + lo[1][e]] = v[1][e];
-                if (WIDE) {
+                if constexpr (WIDE) {
                     S.pos[0][at + lo[0][e]] = p[0][e];
-                    S.pos[WIDE][at + lo[1][e]] = p[1][e];
+                    S.pos[1][at + lo[1][e]] = p[1][e];
                 }
             }
         }
@@ -231,7 +237,8 @@ __device__ __forceinline__ void seg_rank(const cd_contact* __restrict__ seg, uin
     }
     // slot r of the sorted array holds the contact at key r's place; the second order lists those slots
     auto placed = [&](int o, uint32_t r) -> uint32_t {
-        return WIDE ? S.pos[o * WIDE][r] : uint32_t(key[o][r]) & ((1u << SEG_POS_BITS) - 1u);
+        if constexpr (WIDE) return S.pos[o][r];
+        else return uint32_t(key[o][r]) & ((1u << SEG_POS_BITS) - 1u);
     };
 #pragma unroll
     for (uint32_t e = 0; e < E; ++e) {
